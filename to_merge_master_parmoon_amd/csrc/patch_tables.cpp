@@ -1,0 +1,274 @@
+// patch_tables.cpp - builds the records of patch_tables.hpp (host code, once per level).
+#include "patch_tables.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <string>
+#include <system_error>
+#include <thread>
+#include <unordered_map>
+
+namespace pmg {
+
+namespace {
+
+constexpr int NU = 27, NP = 4;
+
+// Which copy of the velocity holds a dof after its i-th of m updates in a sweep.  The new value
+// goes to another copy than the old one, so that the patches of the same color still read the
+// old one, and the last update ends in copy 0 again.  A dof of one cell only is updated in
+// place (the caller checks that no other patch of the color reads it).
+int copy_after(int i, int m) {
+  if (m == 1 || i == 0 || i == m) return 0;
+  if (m % 2 == 1 && i == m - 1) return 2;
+  return i % 2;
+}
+
+struct Dofs {   // the colors that update a dof, ascending
+  std::vector<int> ptr, col, cell;
+};
+
+bool color_lists(int n_dof, int per_cell, const std::vector<int> &glob, int n_colors, const int *ptr,
+                 const int *order, Dofs &out) {
+  out.ptr.assign(n_dof + 1, 0);
+  for (int q = 0; q < ptr[n_colors]; ++q)
+    for (int j = 0; j < per_cell; ++j) out.ptr[glob[size_t(order[q]) * per_cell + j] + 1]++;
+  for (int i = 0; i < n_dof; ++i) out.ptr[i + 1] += out.ptr[i];
+  out.col.resize(out.ptr[n_dof]);
+  out.cell.resize(out.ptr[n_dof]);
+  std::vector<int> at(out.ptr.begin(), out.ptr.end() - 1);
+  for (int k = 0; k < n_colors; ++k)
+    for (int q = ptr[k]; q < ptr[k + 1]; ++q)
+      for (int j = 0; j < per_cell; ++j) {
+        const int g = glob[size_t(order[q]) * per_cell + j];
+        // two cells of one color (or one cell twice) on a dof: the updates would not be ordered
+        if (at[g] > out.ptr[g] && out.col[at[g] - 1] == k) return false;
+        out.col[at[g]] = k;
+        out.cell[at[g]++] = order[q];
+      }
+  return true;
+}
+
+struct Scratch {
+  std::vector<int> mark, pmark;   // dof -> place in the halo (valid where stamp matches)
+  std::vector<int> stamp, pstamp;
+  std::vector<int> halo, runs;
+  std::vector<uint32_t> pat;      // the pattern of the cell in work
+};
+
+}  // namespace
+
+void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, const std::vector<int> &pg, int n_colors,
+                        const int *ptr, const int *order, PatchTables &T) {
+  T = PatchTables{};
+  const int n_pos = ptr[n_colors];
+  if (n_pos <= 0 || d->n_pdof % 4 != 0) return;
+  for (int i = 0; i < d->n_udof; ++i)
+    if (d->a_rowptr[i + 1] - d->a_rowptr[i] > PT_ROW || d->bt_rowptr[i + 1] - d->bt_rowptr[i] > PT_BT) return;
+  for (int i = 0; i < d->n_pdof; ++i)
+    if (d->b_rowptr[i + 1] - d->b_rowptr[i] > PT_BT) return;
+  Dofs U, P;
+  if (!color_lists(d->n_udof, NU, ug, n_colors, ptr, order, U)) return;
+  if (!color_lists(d->n_pdof, NP, pg, n_colors, ptr, order, P)) return;
+  for (int i = 0; i < d->n_pdof; ++i)
+    if (P.ptr[i + 1] - P.ptr[i] > 1) return;   // pressures are updated in place
+  for (int i = 0; i < d->n_udof; ++i) {
+    const int m = U.ptr[i + 1] - U.ptr[i];
+    if (m > 1) T.n_buffers = std::max(T.n_buffers, m % 2 ? 3 : 2);
+  }
+  if (long(T.n_buffers) * d->n_udof > 0x7fffffffL / 4) return;
+
+  std::vector<int> color_of(n_pos);
+  for (int k = 0; k < n_colors; ++k)
+    for (int q = ptr[k]; q < ptr[k + 1]; ++q) color_of[q] = k;
+  auto len_a = [&](int r) { return d->a_rowptr[r + 1] - d->a_rowptr[r]; };
+  auto len_bt = [&](int r) { return r < d->n_active ? d->bt_rowptr[r + 1] - d->bt_rowptr[r] : 0; };
+  // local rows by decreasing length into the velocity quads, heaviest wavefronts last filled
+  static const int quad_order[7] = {0, 2, 4, 5, 6, 7, 3};
+  auto row_places = [&](const int *u, int (&place)[NU]) {
+    int idx[NU];
+    for (int j = 0; j < NU; ++j) idx[j] = j;
+    std::stable_sort(idx, idx + NU, [&](int a, int b) {
+      const int la = len_a(u[a]), lb = len_a(u[b]);
+      return la != lb ? la > lb : len_bt(u[a]) > len_bt(u[b]);
+    });
+    for (int k = 0; k < NU; ++k) place[idx[k]] = quad_order[k / 4] * 4 + k % 4;
+  };
+  using G = PatchShape<true>;
+  using R = PatchShape<false>;
+  T.grid = true;
+  for (int q = 0; q < n_pos && T.grid; ++q) {
+    const int *u = &ug[size_t(order[q]) * NU];
+    int place[NU];
+    row_places(u, place);
+    for (int j = 0; j < NU; ++j) {
+      const int qd = place[j] / 4;
+      T.grid = T.grid && len_a(u[j]) <= 16 * G::a(qd) && len_bt(u[j]) <= 16 * G::bt(qd);
+    }
+  }
+  int off_a[8], off_bt[8];
+  for (int qd = 0; qd < 8; ++qd) {
+    off_a[qd] = T.grid ? G::off_a(qd) : R::off_a(qd);
+    off_bt[qd] = T.grid ? G::off_bt(qd) : R::off_bt(qd);
+  }
+  const int own = T.grid ? G::own : R::own, words = T.grid ? G::words : R::words;
+
+  // records with a fixed largest halo, then packed to the level's own largest halo
+  const int wide = PR_HALO + PT_HALO;
+  std::vector<int> rec(size_t(n_pos) * wide, 0);
+  std::unordered_map<std::string, int> known;   // pattern words -> number in the order of arrival
+  std::mutex known_mu;
+  std::atomic<bool> ok{true};
+  std::atomic<int> next{0};
+  std::atomic<int> hmax{0};
+  auto work_cells = [&] {
+    Scratch W;
+    W.mark.assign(d->n_udof, 0);
+    W.stamp.assign(d->n_udof, -1);
+    W.pmark.assign(d->n_pdof / 4, 0);
+    W.pstamp.assign(d->n_pdof / 4, -1);
+    for (;;) {
+      const int q0 = next.fetch_add(64), q1 = std::min(n_pos, q0 + 64);
+      if (q0 >= n_pos || !ok) return;
+      for (int q = q0; q < q1 && ok; ++q) {
+        const int cell = order[q], color = color_of[q];
+        const int *u = &ug[size_t(cell) * NU], *p = &pg[size_t(cell) * NP];
+        W.halo.clear();
+        W.runs.clear();
+        auto see = [&](int g) {
+          if (W.stamp[g] != q) {
+            W.stamp[g] = q;
+            W.halo.push_back(g);
+          }
+        };
+        for (int j = 0; j < NU; ++j) {
+          see(u[j]);
+          for (int k = d->a_rowptr[u[j]]; k < d->a_rowptr[u[j] + 1]; ++k) see(d->a_kcol[k]);
+          if (u[j] < d->n_active)
+            for (int k = d->bt_rowptr[u[j]]; k < d->bt_rowptr[u[j] + 1]; ++k) {
+              const int g = d->bt_kcol[k] / 4;
+              if (W.pstamp[g] != q) {
+                W.pstamp[g] = q;
+                W.runs.push_back(g);
+              }
+            }
+        }
+        for (int j = 0; j < NP; ++j)
+          for (int k = d->b_rowptr[p[j]]; k < d->b_rowptr[p[j] + 1]; ++k) see(d->b_kcol[k]);
+        const int nh = int(W.halo.size()), nr = int(W.runs.size());
+        if (nh > PT_HALO || nr > PT_RUNS) {
+          ok = false;
+          return;
+        }
+        std::sort(W.halo.begin(), W.halo.end());
+        std::sort(W.runs.begin(), W.runs.end());
+        int h = hmax.load();
+        while (nh > h && !hmax.compare_exchange_weak(h, nh)) {
+        }
+        int *rc = &rec[size_t(q) * wide];
+        for (int i = 0; i < nh; ++i) {
+          const int g = W.halo[i];
+          W.mark[g] = i;
+          const int b = U.ptr[g], m = U.ptr[g + 1] - b;
+          int k = 0;
+          while (k < m && U.col[b + k] < color) ++k;
+          // updated in place by another patch of this color: its old value would be lost
+          if (m == 1 && U.col[b] == color && U.cell[b] != cell) ok = false;
+          rc[PR_HALO + i] = copy_after(k, m) * d->n_udof + g;
+        }
+        for (int i = 0; i < nr; ++i) {
+          const int g = W.runs[i];
+          W.pmark[g] = i;
+          rc[PR_RUN + i] = 4 * g;
+          for (int j = 4 * g; j < 4 * g + 4; ++j)
+            if (P.ptr[j + 1] > P.ptr[j] && P.col[P.ptr[j]] == color && P.cell[P.ptr[j]] != cell) ok = false;
+        }
+        for (int j = 0; j < NU; ++j) {
+          const int b = U.ptr[u[j]], m = U.ptr[u[j] + 1] - b;
+          int k = 0;
+          while (k < m && U.col[b + k] < color) ++k;
+          rc[PR_OUT + j] = copy_after(k + 1, m) * d->n_udof + u[j];
+          rc[PR_DOFS + j] = u[j];
+        }
+        for (int j = 0; j < NP; ++j) rc[PR_DOFS + NU + j] = p[j];
+        rc[PR_HEAD + 1] = nh;
+        rc[PR_HEAD + 2] = nr;
+        // rows and their column positions
+        for (int e = 0; e < 32; ++e) rc[PR_DESC + 4 * e + 2] = PT_NOROW << 16;
+        W.pat.assign(words, 0u);
+        auto put = [&](int off, int e, int j, int pos) {   // entry j of the row at place e
+          const int step = j / 16, lane = (e % 4) * 16 + j % 16;
+          W.pat[size_t(off + step / 2) * 64 + lane] |= uint32_t(pos) << (16 * (step & 1));
+        };
+        auto desc = [&](int e, int k0, int q0b, int n, int m, int row, int g) {
+          int *o = rc + PR_DESC + 4 * e;
+          o[0] = k0;
+          o[1] = q0b;
+          o[2] = n | m << 8 | row << 16;
+          o[3] = g;
+        };
+        int place[NU];
+        row_places(u, place);
+        for (int j = 0; j < NU; ++j) {
+          const int e = place[j], qd = e / 4, g = u[j], k0 = d->a_rowptr[g], n = len_a(g), m = len_bt(g);
+          const int q0b = d->bt_rowptr[g];
+          desc(e, k0, q0b, n, m, j, g);
+          for (int k = 0; k < n; ++k) put(off_a[qd], e, k, W.mark[d->a_kcol[k0 + k]]);
+          for (int k = 0; k < m; ++k) {
+            const int c = d->bt_kcol[q0b + k];
+            put(off_bt[qd], e, k, 4 * W.pmark[c / 4] + c % 4);
+          }
+          W.pat[own + j / 2] |= uint32_t(W.mark[g]) << (16 * (j & 1));
+        }
+        for (int j = 0; j < NP; ++j) {
+          const int e = 4 + j, k0 = d->b_rowptr[p[j]], n = d->b_rowptr[p[j] + 1] - k0;
+          desc(e, k0, 0, n, 0, NU + j, p[j]);
+          for (int k = 0; k < n; ++k) put(off_a[1], e, k, W.mark[d->b_kcol[k0 + k]]);
+        }
+        std::string key(reinterpret_cast<const char *>(W.pat.data()), W.pat.size() * sizeof(uint32_t));
+        std::lock_guard<std::mutex> lk(known_mu);
+        rc[PR_HEAD] = known.emplace(std::move(key), int(known.size())).first->second;
+      }
+    }
+  };
+  auto work = [&] {   // out of memory: the level keeps the two-launch form
+    try {
+      work_cells();
+    } catch (const std::bad_alloc &) {
+      ok = false;
+    }
+  };
+  {
+    const int nt = std::max(1, std::min({8, int(std::thread::hardware_concurrency()), (n_pos + 255) / 256}));
+    std::vector<std::thread> th;
+    try {
+      th.reserve(nt);
+      for (int i = 1; i < nt; ++i) th.emplace_back(work);
+    } catch (const std::system_error &) {   // no more threads: this one does the rest
+    }
+    work();
+    for (auto &t : th) t.join();
+  }
+  if (!ok) return;
+  // the patterns in the order of their first cell, whatever order the threads met them in
+  std::vector<int> number(known.size(), -1);
+  std::vector<const std::string *> text(known.size());
+  for (const auto &kv : known) text[kv.second] = &kv.first;
+  T.pat.resize(known.size() * size_t(words));
+  for (int q = 0; q < n_pos; ++q) {
+    int &id = rec[size_t(q) * wide + PR_HEAD];
+    if (number[id] < 0) {
+      number[id] = T.n_patterns++;
+      std::memcpy(&T.pat[size_t(number[id]) * words], text[id]->data(), text[id]->size());
+    }
+    id = number[id];
+  }
+  T.stride = (PR_HALO + hmax + 15) / 16 * 16;
+  T.rec.resize(size_t(n_pos) * T.stride);
+  for (int q = 0; q < n_pos; ++q) std::memcpy(&T.rec[size_t(q) * T.stride], &rec[size_t(q) * wide], 4 * std::min(wide, T.stride));
+  T.ok = true;
+}
+
+}  // namespace pmg

@@ -658,6 +658,13 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   }
   if (relax) launch_copy<T>(aux, u, D.n_dof, c->stream);
   const OpView<T> op = opview<T>(D);
+  const int nref = sizeof(T) == 4 ? c->prm.bf16_refine_steps : 0;
+  // one launch per color: residual, local solve and update of a patch by one workgroup, at every
+  // size faster than the two launches (k_patch.hip); these stay for refinement steps, nine
+  // blocks, stored LU factors and levels whose patches fit no record (rows of more than 128
+  // entries, shared pressure dofs, colors that share dofs)
+  const bool fused = ua && D.patch_rec && nref == 0;
+  const bool full = !D.schur;
   for (int col = 0; col < D.n_colors; ++col) {
     const int p0 = D.ptr_colors[col];
     // all patches of the color, or (compacted merged level) those of unfinished problems
@@ -676,6 +683,19 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
       nc = int(D.act_slots_off[col + 1] - D.act_slots_off[col]);
       if (nc == 0) continue;
     }
+    if constexpr (sizeof(T) == 4) {
+      if (fused) {
+        const double sb = full ? double(MINV_STRIDE) : double(SCH_STRIDE);
+        // the rows of the residual, the stored data, the record, the new values
+        const double by = D.res_bytes[1][1][col] * part - nc * (31.0 * 20 + 2 * 85 * 4.0) +
+                          nc * (sb * fb + 4.0 * D.patch_stride + 27 * 16.0 + 32);
+        Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
+        PatchStep P{D.patch_rec, D.patch_pat, slots, op.a1, op.btv, op.bv, f, u, ua, damp, D.patch_stride, D.n_udof,
+                    nc, p0, nc >= XCD_GROUP_MIN && D.tune_res_xcd[1], full, D.patch_grid};
+        launch_patch_step(P, D.minv32, D.minv16, full, c->stream);
+        continue;
+      }
+    }
     {
       const double rb = D.res_bytes[D.a_shared][vs == 8 ? 0 : 1][col] * part;
       Timed tm(c, &c->tm.vanka_res, rb, 0.0, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
@@ -687,7 +707,6 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
     }
     // refinement steps (stored inverses only): the stored FP32 patch matrix read once per
     // patch, one more local residual and product per step
-    const int nref = sizeof(T) == 4 ? c->prm.bf16_refine_steps : 0;
     if (nref > 0 && !D.kref)
       throw Fail{PMG_ERR_NOT_READY, "bf16_refine_steps was set after the set-up: call pmg_refactor"};
     const double kent = D.schur ? double(KREF_BLK) : double(KREF_FULL);
@@ -2217,7 +2236,21 @@ static int add_level(pmg_ctx *c, const pmg_level_desc *d, int *level_out, bool m
         D.minv16 = dalloc<uint16_t>(c, minvn);
         launch_fill<uint16_t>(D.minv16, uint16_t(0), long(minvn), c->stream);
       }
-      if (D.minv32 || D.minv16) D.ua32 = dalloc<float>(c, 4 * size_t(D.n_udof)); else if (c->prm.precision == PMG_PREC_FP32) {
+      if (D.minv32 || D.minv16) {
+        PatchTables T;
+        build_patch_tables(d, ug, pg, nc, D.ptr_colors.data(), reo.data(), T);
+        if (T.ok) {
+          D.patch_rec = dalloc<int>(c, T.rec.size());
+          h2d(c, D.patch_rec, T.rec.data(), T.rec.size());
+          D.patch_pat = dalloc<uint32_t>(c, T.pat.size());
+          h2d(c, D.patch_pat, T.pat.data(), T.pat.size());
+          D.patch_stride = T.stride;
+          D.patch_buffers = T.n_buffers;
+          D.patch_grid = T.grid;
+          PMG_HIP_CHECK(hipStreamSynchronize(c->stream));
+        }
+        D.ua32 = dalloc<float>(c, 4 * size_t(D.n_udof) * D.patch_buffers);
+      } else if (c->prm.precision == PMG_PREC_FP32) {
         D.lu32 = dalloc<float>(c, lun);
         launch_fill<float>(D.lu32, 0.0f, long(lun), c->stream);
       } else {

@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "patch_tables.hpp"
 #include "pmg.h"
 
 namespace pmg {
@@ -167,7 +168,13 @@ struct DevLevel {
   uint16_t *minv16 = nullptr;
   // FP32 sweeps with inverses and the shared block: interleaved copy (u1, u2, u3, 0) of the
   // velocity the residual gathers, built at the sweep start and kept by the local updates
+  // With the patch records below it holds patch_buffers such copies, the current one first.
   float *ua32 = nullptr;
+  // records of the fused color step (null: the two-launch form)
+  int *patch_rec = nullptr;
+  uint32_t *patch_pat = nullptr;
+  int patch_stride = 0, patch_buffers = 1;
+  bool patch_grid = false;
   // the patch inverses are stored in the block form (set at every factorization: shared
   // velocity block present)
   bool schur = false;
@@ -375,6 +382,22 @@ void launch_row_blocked(const DevLevel &L, T *av, T *bv, T *btv, hipStream_t s);
 // true when the level's A blocks have the shared form of OpView::a1 (part: 256 doubles of
 // device scratch; synchronizes the stream)
 bool shared_velocity_block(const DevLevel &L, double *part, hipStream_t s);
+// one color of the FP32 sweep with stored inverses and the shared block in one launch
+struct PatchStep {
+  const int *rec;             // records of the level (patch_tables.hpp)
+  const uint32_t *pat;
+  const int *slots;           // positions of the patches relative to pos0 (null: 0 .. ncells-1)
+  const float *a1, *btv, *bv; // operator values of the streamed rows
+  const float *f;
+  float *u, *ua;              // pressure (and, mirror, velocity); the copies of the velocity
+  float damp;
+  int stride, N, ncells, pos0;
+  int grouped;                // 1: consecutive patches of the color per XCD
+  int mirror;                 // 1: u takes the new velocity too
+  int grid;                   // PatchShape<true>, else <false>
+};
+// full: the stored data is the full inverse, else the block form
+void launch_patch_step(const PatchStep &P, const float *stored32, const uint16_t *stored16, bool full, hipStream_t s);
 template <typename T, typename F>
 // ncells patches of one color: slots (may be null: 0..ncells-1) are their positions
 // relative to pos0 and their local residual slots

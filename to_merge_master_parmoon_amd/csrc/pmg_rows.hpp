@@ -11,13 +11,25 @@
 
 namespace pmg {
 
-// sum over the 16 lanes of a row group (every lane gets the total)
+// v of the lane N places round in the group of 16
+template <int N>
+__device__ inline float ror16(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ inline double ror16(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + N, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + N, 0xf, 0xf, true));
+}
+// sum over the 16 lanes of a row group (every lane gets the total), by rotations inside the
+// group: after adding the lane 8 places round the values repeat every 8 lanes, so the lane 4
+// places round is the one across, and so on; no LDS permutes in the chain
 template <typename T>
 __device__ inline T red16(T v) {
-  v += __shfl_xor(v, 8, 16);
-  v += __shfl_xor(v, 4, 16);
-  v += __shfl_xor(v, 2, 16);
-  v += __shfl_xor(v, 1, 16);
+  v += ror16<8>(v);
+  v += ror16<4>(v);
+  v += ror16<2>(v);
+  v += ror16<1>(v);
   return v;
 }
 
