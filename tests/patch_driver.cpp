@@ -56,11 +56,13 @@ static void plain(const Sys &S, int nc, const int *ptr, const int *order, std::v
 
 // the sweep from the records
 static void records(const Sys &S, const PatchTables &T, int nc, const int *ptr, std::vector<double> &ub,
-                    std::vector<double> &p, std::mt19937 &rng) {
+                    std::vector<double> &p, std::mt19937 &rng, bool fp64) {
   const pmg_level_desc &d = *S.d;
   const long nb = long(T.n_buffers) * d.n_udof;
-  const int words = T.grid ? PatchShape<true>::words : PatchShape<false>::words;
-  const int p_own = T.grid ? PatchShape<true>::own : PatchShape<false>::own;
+  const int words = fp64 ? (T.grid ? PatchShape64<true>::words : PatchShape64<false>::words)
+                         : T.grid ? PatchShape<true>::words : PatchShape<false>::words;
+  const int p_own = fp64 ? (T.grid ? PatchShape64<true>::own : PatchShape64<false>::own)
+                         : T.grid ? PatchShape<true>::own : PatchShape<false>::own;
   for (int k = 0; k < nc; ++k) {
     std::vector<int> at;
     for (int q = ptr[k]; q < ptr[k + 1]; ++q) at.push_back(q);
@@ -83,15 +85,30 @@ static void records(const Sys &S, const PatchTables &T, int nc, const int *ptr, 
       for (int e = 0; e < 32; ++e) {
         const int *dc = rc + PR_DESC + 4 * e, qd = e / 4;
         const int n = dc[2] & 255, m = (dc[2] >> 8) & 255, row = (dc[2] >> 16) & 255;
-        const int sa = T.grid ? PatchShape<true>::a(qd) : PatchShape<false>::a(qd);
-        const int sb = T.grid ? PatchShape<true>::bt(qd) : PatchShape<false>::bt(qd);
-        const int off_a = T.grid ? PatchShape<true>::off_a(qd) : PatchShape<false>::off_a(qd);
-        const int off_bt = T.grid ? PatchShape<true>::off_bt(qd) : PatchShape<false>::off_bt(qd);
+        const int sa = fp64 ? 4 * (T.grid ? PatchShape64<true>::a(qd) : PatchShape64<false>::a(qd))
+                            : T.grid ? PatchShape<true>::a(qd) : PatchShape<false>::a(qd);
+        const int sb = fp64 ? (qd == 1 ? 0 : 4) : T.grid ? PatchShape<true>::bt(qd) : PatchShape<false>::bt(qd);
+        const int off_a = fp64 ? (T.grid ? PatchShape64<true>::off_a(qd) : PatchShape64<false>::off_a(qd))
+                               : 64 * (T.grid ? PatchShape<true>::off_a(qd) : PatchShape<false>::off_a(qd));
+        const int off_bt = fp64 ? (T.grid ? PatchShape64<true>::off_bt(qd) : PatchShape64<false>::off_bt(qd))
+                                : 64 * (T.grid ? PatchShape<true>::off_bt(qd) : PatchShape<false>::off_bt(qd));
         CHECK((n + 15) / 16 <= sa && (m + 15) / 16 <= sb);
-        auto pos = [&](int off, int j) {
-          const size_t w = size_t(off + j / 32) * 64 + (e % 4) * 16 + j % 16;
+        // position of entry j of a row of len entries: in FP64 the kernel's lane reads the four
+        // entries from the start of its window on
+        auto pos = [&](int off, int j, int len) {
+          size_t w;
+          int half;
+          if (fp64) {
+            const int lane = j % 64 / 4, jb = j / 4 * 4, ld = len >= 4 ? std::min(jb, len - 4) : 0, u = j - ld;
+            CHECK(u >= 0 && u < 4 && ld + u >= jb);
+            w = size_t(off) + 2 * (64 * (j / 64) + (e % 4) * 16 + lane) + u / 2;
+            half = u & 1;
+          } else {
+            w = size_t(off) + 64 * (j / 32) + (e % 4) * 16 + j % 16;
+            half = (j / 16) & 1;
+          }
           CHECK(w < size_t(p_own));
-          return int((pat[w] >> (16 * ((j / 16) & 1))) & 0xffffu);
+          return int((pat[w] >> (16 * half)) & 0xffffu);
         };
         if (row == PT_NOROW) {
           CHECK(n == 0 && m == 0);
@@ -101,8 +118,8 @@ static void records(const Sys &S, const PatchTables &T, int nc, const int *ptr, 
           CHECK(row >= 27 && row < 31 && dc[0] + n <= d.b_nnz && dc[3] >= 0 && dc[3] < d.n_pdof);
           double s = 0;
           for (int j = 0; j < n; ++j) {
-            CHECK(pos(off_a, j) < nh);
-            for (int c = 0; c < 3; ++c) s += d.b[c][dc[0] + j] * hv[3 * pos(off_a, j) + c];
+            CHECK(pos(off_a, j, n) < nh);
+            for (int c = 0; c < 3; ++c) s += d.b[c][dc[0] + j] * hv[3 * pos(off_a, j, n) + c];
           }
           r[81 + row - 27] = 1.0 - s;
           continue;
@@ -110,12 +127,12 @@ static void records(const Sys &S, const PatchTables &T, int nc, const int *ptr, 
         CHECK(row < 27 && dc[0] + n <= d.a_nnz && dc[1] + m <= d.bt_nnz && dc[3] >= 0 && dc[3] < d.n_udof);
         double s[3] = {0, 0, 0};
         for (int j = 0; j < n; ++j) {
-          CHECK(pos(off_a, j) < nh);
-          for (int c = 0; c < 3; ++c) s[c] += d.a[0][dc[0] + j] * hv[3 * pos(off_a, j) + c];
+          CHECK(pos(off_a, j, n) < nh);
+          for (int c = 0; c < 3; ++c) s[c] += d.a[0][dc[0] + j] * hv[3 * pos(off_a, j, n) + c];
         }
         for (int j = 0; j < m; ++j) {
-          CHECK(pos(off_bt, j) < 4 * nr);
-          for (int c = 0; c < 3; ++c) s[c] += d.bt[c][dc[1] + j] * hp[pos(off_bt, j)];
+          CHECK(pos(off_bt, j, m) < 4 * nr);
+          for (int c = 0; c < 3; ++c) s[c] += d.bt[c][dc[1] + j] * hp[pos(off_bt, j, m)];
         }
         for (int c = 0; c < 3; ++c) r[27 * c + row] = 1.0 - s[c];
       }
@@ -132,7 +149,7 @@ static void records(const Sys &S, const PatchTables &T, int nc, const int *ptr, 
   }
 }
 
-static void run(const char *name, pmgp_problem *prob, int level, int mode) {
+static void run(const char *name, pmgp_problem *prob, int level, int mode, bool fp64) {
   pmg_level_desc d;
   pmgp_level_desc(prob, level, &d);
   Sys S{&d, {}, {}};
@@ -165,7 +182,7 @@ static void run(const char *name, pmgp_problem *prob, int level, int mode) {
     std::sort(order.begin(), order.begin() + ptr[1]);
   }
   PatchTables T;
-  build_patch_tables(&d, S.ug, S.pg, nc, ptr.data(), order.data(), T);
+  build_patch_tables(&d, S.ug, S.pg, nc, ptr.data(), order.data(), fp64, T);
   if (mode == 3) {
     CHECK(!T.ok);
     return;
@@ -181,7 +198,7 @@ static void run(const char *name, pmgp_problem *prob, int level, int mode) {
   std::copy(u.begin(), u.end(), b.begin());
   for (int sweep = 0; sweep < 2; ++sweep) {
     plain(S, nc, ptr.data(), order.data(), u, p);
-    records(S, T, nc, ptr.data(), b, q, rng);
+    records(S, T, nc, ptr.data(), b, q, rng, fp64);
   }
   double err = 0, nrm = 0;
   for (size_t i = 0; i < u.size(); ++i) { const double e = std::fabs(u[i] - b[i]); CHECK(e == e); err = std::max(err, e); nrm = std::max(nrm, std::fabs(u[i])); }
@@ -204,7 +221,7 @@ int main() {
     pmgp_problem *P = nullptr;
     if (pmgp_create(&c, &P)) { printf("create failed\n"); return 1; }
     for (int l = 0; l < s.levels; ++l)
-      for (int mode = 0; mode < 5; ++mode) run(s.name, P, l, mode);
+      for (int mode = 0; mode < 10; ++mode) run(s.name, P, l, mode % 5, mode >= 5);
     pmgp_destroy(P);
   }
   printf(bad ? "FAIL %d\n" : "OK\n", bad);

@@ -18,6 +18,7 @@
 // stored data), the two launches before and this one: 32^3 30.5 + 8.8 -> 20.4 us, 24^3 (full
 // inverses) 14.4 + 8.7 -> 13.0 us, 16^3 6.4 + 4.9 -> 6.2 us, 8^3 4.7 + 4.4 -> 4.4 us; the same
 // sums in the same order, so the same results bit for bit.
+#include "lu_sweeps.hpp"
 #include "pmg_internal.hpp"
 #include "pmg_rows.hpp"
 
@@ -304,24 +305,29 @@ __device__ __forceinline__ void patch_wave(const PatchStep &P, const F *__restri
   }
 }
 
+// the patch of this workgroup (-1: none)
+template <class Step>
+__device__ __forceinline__ int patch_slot(const Step &P) {
+  int slot = blockIdx.x;
+  if (P.grouped) {
+    // workgroup b runs on XCD b % 8 and takes its share of the b % 8-th eighth of the color's
+    // consecutive cells, so that an XCD's L2 holds the vectors of one compact part of the mesh
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const int b0 = int(long(P.ncells) * x / 8), b1 = int(long(P.ncells) * (x + 1) / 8);
+    if (k >= b1 - b0) return -1;
+    slot = b0 + k;
+  }
+  return P.slots ? P.slots[slot] : slot;
+}
+
 // FULL: stored 85 x 85 inverse (minv layout), else the block form (SCH_* layout).  GRID: shape
 // of the records' patterns.
 template <typename F, bool FULL, bool GRID>
 __global__ __launch_bounds__(256) void k_patch_step(PatchStep P, const F *__restrict__ stored) {
   __shared__ __align__(16) PatchLds<F, FULL> S;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l64 = threadIdx.x & 63;
-  int slot;
-  if (P.grouped) {
-    // workgroup b runs on XCD b % 8 and takes its share of the b % 8-th eighth of the color's
-    // consecutive cells, so that an XCD's L2 holds the vectors of one compact part of the mesh
-    const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const int b0 = int(long(P.ncells) * x / 8), b1 = int(long(P.ncells) * (x + 1) / 8);
-    if (k >= b1 - b0) return;
-    slot = b0 + k;
-  } else {
-    slot = blockIdx.x;
-  }
-  if (P.slots) slot = P.slots[slot];
+  const int slot = patch_slot(P);
+  if (slot < 0) return;
   const long pos = long(P.pos0) + slot;
   if (wave == 0)
     patch_wave<F, FULL, GRID, 0>(P, stored, pos, l64, S);
@@ -333,7 +339,240 @@ __global__ __launch_bounds__(256) void k_patch_step(PatchStep P, const F *__rest
     patch_wave<F, FULL, GRID, 3>(P, stored, pos, l64, S);
 }
 
+// ------------------------------------------------------------------ FP64
+// The same step with the FP64 operator and the stored LU factors of dgetf2 (k_patch_lu).  The
+// velocity stays in the component vectors: copy 0 is u itself, the others follow in P.alt.
+// Bounds: small colors the chain of 170 steps of the two sweeps (lu_sweeps.hpp); large ones the
+// stream of factors and rows, 100 KB per patch (226 registers allow two workgroups per CU, whose
+// loads in flight cover the latency).  Residual and solve launches before -> this one, per color:
+// 8^3 5.8 + 9.5 -> 9.2 us, 16^3 11.5 + 13.8 -> 15.8 us, 12 x 16 x 20 10.9 + 13.2 -> 14.8 us; the
+// set-up and solve at 32^3 72.0 -> 54.7 ms.  The same results bit for bit.
+__device__ __forceinline__ double *velocity_at(const PatchStep64 &P, int loc) {
+  double *p = P.u + loc;
+  if (loc >= P.N) {
+    loc -= P.N;
+    p = P.alt + loc;
+    if (loc >= P.N) p = P.alt + 2L * P.N + loc;   // 3 N + (loc - N)
+  }
+  return p;
+}
+
+// four consecutive entries from p on (8-byte aligned)
+__device__ __forceinline__ void ld4d(const double *p, double (&o)[4]) { ld4(p, o); }
+__device__ __forceinline__ int window(int jb, int n) { return n >= 4 ? min(jb, n - 4) : 0; }
+
+template <class SH, int QD>
+struct Row64 {
+  static constexpr int NB = QD == 1 ? 0 : SH::a(QD), OA = SH::off_a(QD), OB = SH::off_bt(QD);
+  int n, m, row;
+  double a[NB > 0 ? NB : 1][4], b[3][4], f;
+  uint2 ia[NB > 0 ? NB : 1], ib;
+  int perm;
+  __device__ __forceinline__ void load(const PatchStep64 &P, const int4 d, const uint32_t *__restrict__ pat,
+                                       const uint8_t *__restrict__ ip, int l64) {
+    const int lane = l64 & 15;
+    n = d.z & 255;
+    m = (d.z >> 8) & 255;
+    row = (d.z >> 16) & 255;
+    if constexpr (QD == 1) {
+      // pressure row: the three blocks of B
+      ib = reinterpret_cast<const uint2 *>(pat + OA)[l64];
+      const double *v = P.bv + 3L * d.x + window(4 * lane, n);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) ld4d(v + c * n, b[c]);
+      f = P.f[3L * P.N + d.w];
+      perm = ip[min(row + 2 * NU_LOC, NLOC - 1)];
+    } else {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) ia[k] = reinterpret_cast<const uint2 *>(pat + OA + 128 * k)[l64];
+      ib = reinterpret_cast<const uint2 *>(pat + OB)[l64];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) ld4d(P.a1 + d.x + window(64 * k + 4 * lane, n), a[k]);
+      const double *w = P.btv + 3L * d.y + window(4 * lane, m);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) ld4d(w + c * m, b[c]);
+      f = P.f[long(lane < 3 ? lane : 0) * P.N + d.w];
+      perm = ip[min(row + NU_LOC * (lane < 3 ? lane : 0), NLOC - 1)];
+    }
+  }
+  static __device__ __forceinline__ int at(uint2 w, int u) { return ((u < 2 ? w.x : w.y) >> (16 * (u & 1))) & 0xffffu; }
+  // the entries of a lane's window that are its own (row_window)
+  static __device__ __forceinline__ bool own(int jb, int len, int u) {
+    const int e = window(jb, len) + u;
+    return e >= jb && e < len;
+  }
+  // sums in the order of row_a1_v, row_bt_v and row_b_v
+  __device__ __forceinline__ void residual(const double *hv, const double *hp, double *rs, int l64) const {
+    const int lane = l64 & 15;
+    if constexpr (QD == 1) {
+      double s = 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double *y = hv + at(ib, u);
+        const bool ok = own(4 * lane, n, u);
+        const double z1 = ok ? y[0] : 0.0, z2 = ok ? y[PT_HALO] : 0.0, z3 = ok ? y[2 * PT_HALO] : 0.0;
+        // contracted as row_b_v is compiled in k_vanka_res
+        s += fma(b[2][u], z3, u == 0 ? fma(b[1][u], z2, b[0][u] * z1) : fma(b[0][u], z1, b[1][u] * z2));
+      }
+      s = red16(s);
+      if (lane == 0 && row != PT_NOROW) rs[perm] = f - s;
+    } else {
+      double s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const double *y = hv + at(ia[k], u);
+          const double w = own(64 * k + 4 * lane, n, u) ? a[k][u] : 0.0;
+          s1 += w * y[0];
+          s2 += w * y[PT_HALO];
+          s3 += w * y[2 * PT_HALO];
+        }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double z = own(4 * lane, m, u) ? hp[at(ib, u)] : 0.0;
+        s1 += b[0][u] * z;
+        s2 += b[1][u] * z;
+        s3 += b[2][u] * z;
+      }
+      s1 = red16(s1);
+      s2 = red16(s2);
+      s3 = red16(s3);
+      if (lane < 3 && row != PT_NOROW) rs[perm] = f - (lane == 0 ? s1 : lane == 1 ? s2 : s3);
+    }
+  }
+};
+
+struct Patch64Lds {
+  double hv[3 * PT_HALO], hp[4 * PT_RUNS], rs[RLOC_STRIDE];
+  v4u fac[32 + 64 * 29];   // a factor part after 64 entries of padding (k_vanka_solve)
+};
+
+template <bool GRID, int W>
+__device__ __forceinline__ void patch_wave64(const PatchStep64 &P, long pos, int l64, Patch64Lds &S) {
+  using SH = PatchShape64<GRID>;
+  // 16-byte vectors of the two factor parts, dealt to the four wavefronts in runs of 64
+  constexpr int RL = 28, RU = 29, NL = (RL - W + 3) / 4, NU = (RU - W + 3) / 4;
+  static_assert(64 * RL * 2 >= LU_L && 64 * RU * 2 >= LU_U, "factor parts");
+  static_assert(lu_uoff(NLOC - 1) + 127 < 2 * 64 * RU, "the sweeps read past the copy");
+  const int t = 64 * W + l64;
+  const int *__restrict__ rc = P.rec + pos * P.stride;
+  const int pid = rc[PR_HEAD];
+  const int nh = P.stride - PR_HALO;
+  const int loc0 = rc[PR_HALO + min(t, nh - 1)];
+  int loc1 = 0, run = 0;
+  if constexpr (W < 2) {
+    loc1 = rc[PR_HALO + min(t + 256, nh - 1)];
+    run = rc[PR_RUN + t / 4];
+  }
+  const int4 *__restrict__ ds = reinterpret_cast<const int4 *>(rc + PR_DESC) + 8 * W + (l64 >> 4);
+  const int4 d0 = ds[0], d1 = ds[4];
+  const uint8_t *__restrict__ ip = P.invperm + pos * PERM_STRIDE;
+  // wavefront 0 solves: lane i owns rows i and 64 + i; rows c * 27 + j of dof j, 81 + k of
+  // pressure dof k
+  int out0 = 0, out1 = 0, own0 = 0, own1 = 0;
+  const bool two = l64 < NLOC - 64;
+  const int c0 = l64 / NU_LOC, j0 = l64 - c0 * NU_LOC;             // row l64 < 64
+  const int i1 = min(64 + l64, NLOC - 1), j1 = i1 - 2 * NU_LOC;    // row 64 + l64: component 2 or pressure
+  if constexpr (W == 0) {
+    out0 = rc[PR_OUT + j0];
+    out1 = j1 < NU_LOC ? rc[PR_OUT + j1] : rc[PR_DOFS + j1];
+  }
+  const uint32_t *__restrict__ pat = P.pat + long(pid) * SH::words;
+  const double *const q0 = velocity_at(P, loc0);
+  const double h0[3] = {q0[0], q0[P.N], q0[2L * P.N]};
+  double h1[3] = {0.0, 0.0, 0.0}, hq = 0.0;
+  if constexpr (W < 2) {
+    const double *const q1 = velocity_at(P, loc1);
+    h1[0] = q1[0];
+    h1[1] = q1[P.N];
+    h1[2] = q1[2L * P.N];
+    hq = P.u[3L * P.N + run + t % 4];
+  }
+  Row64<SH, 2 * W> A;
+  Row64<SH, 2 * W + 1> B;
+  A.load(P, d0, pat, ip, l64);
+  B.load(P, d1, pat, ip, l64);
+  if constexpr (W == 0) {
+    own0 = (pat[SH::own + j0 / 2] >> (16 * (j0 & 1))) & 0xffffu;
+    own1 = (pat[SH::own + min(j1, NU_LOC - 1) / 2] >> (16 * (j1 & 1))) & 0xffffu;
+  }
+  double v1 = 0.0;
+  if constexpr (W == 0) v1 = P.u[3L * P.N + (j1 < NU_LOC ? 0 : out1)];   // (velocity rows: unused)
+  // the factors last: they are needed last
+  const v4u *__restrict__ gL = reinterpret_cast<const v4u *>(P.lu + pos * LU_STRIDE);
+  const v4u *__restrict__ gU = reinterpret_cast<const v4u *>(P.lu + pos * LU_STRIDE + LU_UOFF);
+  v4u rL[NL], rU[NU];
+#pragma unroll
+  for (int q = 0; q < NL; ++q) rL[q] = gL[l64 + 64 * (4 * q + W)];
+#pragma unroll
+  for (int q = 0; q < NU; ++q) rU[q] = gU[l64 + 64 * (4 * q + W)];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) S.hv[c * PT_HALO + t] = h0[c];
+  if constexpr (W < 2) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) S.hv[c * PT_HALO + t + 256] = h1[c];
+    S.hp[t] = hq;
+  }
+  patch_barrier();
+  A.residual(S.hv, S.hp, S.rs, l64);
+  B.residual(S.hv, S.hp, S.rs, l64);
+  v4u *const s4 = S.fac + 32;
+#pragma unroll
+  for (int q = 0; q < NL; ++q) s4[l64 + 64 * (4 * q + W)] = rL[q];
+  patch_barrier();
+  // the sweeps of k_vanka_solve, on wavefront 0; the others put the U part in place between them
+  const double *const fac = reinterpret_cast<const double *>(s4);
+  double x0 = 0.0, x1 = 0.0;
+  if constexpr (W == 0) {
+    x0 = S.rs[l64];
+    x1 = two ? S.rs[64 + l64] : 0.0;
+    lower_sweep<double, double>(fac, l64, x0, x1);
+  }
+  patch_barrier();
+#pragma unroll
+  for (int q = 0; q < NU; ++q) s4[l64 + 64 * (4 * q + W)] = rU[q];
+  patch_barrier();
+  if constexpr (W == 0) {
+    upper_sweep<double, double>(fac, l64, two, x0, x1);
+    velocity_at(P, out0)[long(c0) * P.N] = S.hv[c0 * PT_HALO + own0] + P.damp * x0;
+    if (two) {
+      if (j1 < NU_LOC)
+        velocity_at(P, out1)[2L * P.N] = S.hv[2 * PT_HALO + own1] + P.damp * x1;
+      else
+        P.u[3L * P.N + out1] = v1 + P.damp * x1;
+    }
+  }
+}
+
+template <bool GRID>
+__global__ __launch_bounds__(256) void k_patch_step64(PatchStep64 P) {
+  __shared__ Patch64Lds S;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l64 = threadIdx.x & 63;
+  const int slot = patch_slot(P);
+  if (slot < 0) return;
+  const long pos = long(P.pos0) + slot;
+  if (wave == 0)
+    patch_wave64<GRID, 0>(P, pos, l64, S);
+  else if (wave == 1)
+    patch_wave64<GRID, 1>(P, pos, l64, S);
+  else if (wave == 2)
+    patch_wave64<GRID, 2>(P, pos, l64, S);
+  else
+    patch_wave64<GRID, 3>(P, pos, l64, S);
+}
+
 }  // namespace
+
+void launch_patch_step64(const PatchStep64 &P, hipStream_t s) {
+  if (P.ncells <= 0) return;
+  const int grid = P.grouped ? 8 * ((P.ncells + 7) / 8) : P.ncells;
+  if (P.grid)
+    k_patch_step64<true><<<grid, 256, 0, s>>>(P);
+  else
+    k_patch_step64<false><<<grid, 256, 0, s>>>(P);
+  PMG_HIP_CHECK(hipGetLastError());
+}
 
 void launch_patch_step(const PatchStep &P, const float *stored32, const uint16_t *stored16, bool full, hipStream_t s) {
   if (P.ncells <= 0) return;

@@ -13,6 +13,7 @@
 // The factorization and the sweeps perform the same fma/div sequence as the FP64 oracle
 // (dgetf2 pivoting, reciprocal scaling, column-oriented dtrsm), so FP64 factors and
 // local solves agree with it bit for bit.
+#include "lu_sweeps.hpp"
 #include "pmg_internal.hpp"
 #include "pmg_rows.hpp"
 
@@ -22,35 +23,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));   // MFMA f32 accumulator
 
 namespace {
 
-
-__device__ inline double bcast(double v, int lane) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-  return __hiloint2double(hi, lo);
-}
-__device__ inline float bcast(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
-__device__ inline double tfma(double a, double b, double c) { return fma(a, b, c); }
-__device__ inline float tfma(float a, float b, float c) { return fmaf(a, b, c); }
-
-template <typename T, typename F>
-struct Ld;
-template <typename T>
-struct Ld<T, T> {
-  static __device__ inline T get(const T *p, int i) { return p[i]; }
-};
-template <>
-struct Ld<float, double> {
-  static __device__ inline float get(const double *p, int i) { return float(p[i]); }
-};
-template <>
-struct Ld<float, uint16_t> {
-  static __device__ inline float get(const uint16_t *p, int i) {
-    return __uint_as_float(uint32_t(p[i]) << 16);
-  }
-};
 
 // One workgroup per patch position (cells in color order).  The local matrix is the
 // System[col*85+row] of NSE_MGLevel4.C:1066-1290 (velocity rows j, j+27, j+54, pressure
@@ -1037,59 +1009,13 @@ __global__ __launch_bounds__(64) void k_vanka_solve(const F *__restrict__ lu, co
   if constexpr (REG) {
     sweeps_in_registers<T, F>(s4, sl0, sl1, rU, lane, two, x0, x1);
   } else {
-    // unit lower sweep (dtrsm L, column oriented); L(r,k) at lu_loff(k) + r - k - 1.  Row
-    // 64+lane is below every k < 64, row lane is above every k >= 64, so per step only one
-    // of the two rows needs the "below the pivot" test.
-#pragma unroll
-    for (int k = 0; k < NLOC - 1; ++k) {
-      const int o = lu_loff(k) - k - 1;
-      if (k < 64) {
-        const T bk = bcast(x0, k);
-        const T l0 = Ld<T, F>::get(sl0, o), l1 = Ld<T, F>::get(sl1, o);
-        const T y0 = tfma(-bk, l0, x0);
-        x0 = lane > k ? y0 : x0;
-        x1 = tfma(-bk, l1, x1);  // lanes without a second row carry an unused value
-      } else {
-        const T bk = bcast(x1, k - 64);
-        const T l1 = Ld<T, F>::get(sl1, o);
-        const T y1 = tfma(-bk, l1, x1);
-        x1 = lane + 64 > k ? y1 : x1;
-      }
-    }
+    const F *const fac = reinterpret_cast<const F *>(s4);
+    lower_sweep<T, F>(fac, lane, x0, x1);
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < PS::RU; ++q) s4[lane + 64 * q] = rU[q];
     __syncthreads();
-    // upper sweep (dtrsm U): x_k /= U(k,k), then eliminate column k above the diagonal;
-    // U(r,k) at lu_uoff(k) + r.  Row lane is above every k >= 64, row 64+lane below every
-    // k < 64.
-    // Diagonal of U and its reciprocal per lane, computed in parallel before the chain.  The
-    // quotient x_k / U(k,k) is then q = x r, e = fma(-q, U, x), q' = fma(e, r, q): with r the
-    // correctly rounded reciprocal this is the correctly rounded quotient (Markstein), i.e.
-    // the same value as the division of the column-oriented dtrsm, in three dependent steps.
-    const T dg0 = Ld<T, F>::get(reinterpret_cast<const F *>(s4), lu_uoff(lane) + lane);
-    const T dg1 = two ? Ld<T, F>::get(reinterpret_cast<const F *>(s4), lu_uoff(64 + lane) + 64 + lane) : T(1);
-    const T rc0 = T(1) / dg0, rc1 = T(1) / dg1;
-#pragma unroll
-    for (int k = NLOC - 1; k >= 0; --k) {
-      const int o = lu_uoff(k);
-      if (k >= 64) {
-        T q1 = x1 * rc1;
-        if constexpr (sizeof(T) == 8) q1 = tfma(tfma(-q1, dg1, x1), rc1, q1);
-        const T xk = bcast(q1, k - 64);
-        const T u0 = Ld<T, F>::get(sl0, o), u1 = Ld<T, F>::get(sl1, o);
-        x0 = tfma(-xk, u0, x0);  // every row lane < 64 <= k lies above the pivot
-        const T y1 = tfma(-xk, u1, x1);
-        x1 = (lane + 64 == k) ? xk : (lane + 64 < k ? y1 : x1);
-      } else {
-        T q0 = x0 * rc0;
-        if constexpr (sizeof(T) == 8) q0 = tfma(tfma(-q0, dg0, x0), rc0, q0);
-        const T xk = bcast(q0, k);
-        const T u0 = Ld<T, F>::get(sl0, o);
-        const T y0 = tfma(-xk, u0, x0);
-        x0 = (lane == k) ? xk : (lane < k ? y0 : x0);
-      }
-    }
+    upper_sweep<T, F>(fac, lane, two, x0, x1);
   }
   // u[UDOF] += damp * delta, p[PDOF] += damp * delta
   u[o0] = v0 + damp * x0;

@@ -61,7 +61,7 @@ struct Scratch {
 }  // namespace
 
 void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, const std::vector<int> &pg, int n_colors,
-                        const int *ptr, const int *order, PatchTables &T) {
+                        const int *ptr, const int *order, bool fp64, PatchTables &T) {
   T = PatchTables{};
   const int n_pos = ptr[n_colors];
   if (n_pos <= 0 || d->n_pdof % 4 != 0) return;
@@ -98,6 +98,8 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
   };
   using G = PatchShape<true>;
   using R = PatchShape<false>;
+  using G64 = PatchShape64<true>;
+  using R64 = PatchShape64<false>;
   T.grid = true;
   for (int q = 0; q < n_pos && T.grid; ++q) {
     const int *u = &ug[size_t(order[q]) * NU];
@@ -108,12 +110,13 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
       T.grid = T.grid && len_a(u[j]) <= 16 * G::a(qd) && len_bt(u[j]) <= 16 * G::bt(qd);
     }
   }
-  int off_a[8], off_bt[8];
+  int off_a[8], off_bt[8];   // words
   for (int qd = 0; qd < 8; ++qd) {
-    off_a[qd] = T.grid ? G::off_a(qd) : R::off_a(qd);
-    off_bt[qd] = T.grid ? G::off_bt(qd) : R::off_bt(qd);
+    off_a[qd] = fp64 ? (T.grid ? G64::off_a(qd) : R64::off_a(qd)) : 64 * (T.grid ? G::off_a(qd) : R::off_a(qd));
+    off_bt[qd] = fp64 ? (T.grid ? G64::off_bt(qd) : R64::off_bt(qd)) : 64 * (T.grid ? G::off_bt(qd) : R::off_bt(qd));
   }
-  const int own = T.grid ? G::own : R::own, words = T.grid ? G::words : R::words;
+  const int own = fp64 ? (T.grid ? G64::own : R64::own) : T.grid ? G::own : R::own;
+  const int words = fp64 ? (T.grid ? G64::words : R64::words) : T.grid ? G::words : R::words;
 
   // records with a fixed largest halo, then packed to the level's own largest halo
   const int wide = PR_HALO + PT_HALO;
@@ -198,9 +201,15 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
         // rows and their column positions
         for (int e = 0; e < 32; ++e) rc[PR_DESC + 4 * e + 2] = PT_NOROW << 16;
         W.pat.assign(words, 0u);
-        auto put = [&](int off, int e, int j, int pos) {   // entry j of the row at place e
-          const int step = j / 16, lane = (e % 4) * 16 + j % 16;
-          W.pat[size_t(off + step / 2) * 64 + lane] |= uint32_t(pos) << (16 * (step & 1));
+        auto put = [&](int off, int e, int j, int n, int pos) {   // entry j of n of the row at place e
+          if (fp64) {
+            // entry u of the lane's window, which starts at most n - 4 (row_window)
+            const int lane = j % 64 / 4, jb = j / 4 * 4, first = n >= 4 ? std::min(jb, n - 4) : 0, u = j - first;
+            W.pat[size_t(off) + 2 * (64 * (j / 64) + (e % 4) * 16 + lane) + u / 2] |= uint32_t(pos) << (16 * (u & 1));
+          } else {
+            const int step = j / 16, lane = (e % 4) * 16 + j % 16;
+            W.pat[size_t(off) + 64 * (step / 2) + lane] |= uint32_t(pos) << (16 * (step & 1));
+          }
         };
         auto desc = [&](int e, int k0, int q0b, int n, int m, int row, int g) {
           int *o = rc + PR_DESC + 4 * e;
@@ -215,17 +224,17 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
           const int e = place[j], qd = e / 4, g = u[j], k0 = d->a_rowptr[g], n = len_a(g), m = len_bt(g);
           const int q0b = d->bt_rowptr[g];
           desc(e, k0, q0b, n, m, j, g);
-          for (int k = 0; k < n; ++k) put(off_a[qd], e, k, W.mark[d->a_kcol[k0 + k]]);
+          for (int k = 0; k < n; ++k) put(off_a[qd], e, k, n, W.mark[d->a_kcol[k0 + k]]);
           for (int k = 0; k < m; ++k) {
             const int c = d->bt_kcol[q0b + k];
-            put(off_bt[qd], e, k, 4 * W.pmark[c / 4] + c % 4);
+            put(off_bt[qd], e, k, m, 4 * W.pmark[c / 4] + c % 4);
           }
           W.pat[own + j / 2] |= uint32_t(W.mark[g]) << (16 * (j & 1));
         }
         for (int j = 0; j < NP; ++j) {
           const int e = 4 + j, k0 = d->b_rowptr[p[j]], n = d->b_rowptr[p[j] + 1] - k0;
           desc(e, k0, 0, n, 0, NU + j, p[j]);
-          for (int k = 0; k < n; ++k) put(off_a[1], e, k, W.mark[d->b_kcol[k0 + k]]);
+          for (int k = 0; k < n; ++k) put(off_a[1], e, k, n, W.mark[d->b_kcol[k0 + k]]);
         }
         std::string key(reinterpret_cast<const char *>(W.pat.data()), W.pat.size() * sizeof(uint32_t));
         std::lock_guard<std::mutex> lk(known_mu);

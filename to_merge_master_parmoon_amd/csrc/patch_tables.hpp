@@ -47,19 +47,30 @@ struct PatchShape {
   static constexpr int words = own + 16;                            // of a pattern (14 for the own dofs)
 };
 
+// The same for FP64 rows, whose lanes take four consecutive entries of every 64 (row_window): two
+// words of two positions per lane and batch of 64, at off_a(quad) + 2 * (64 * batch + lane).
+template <bool GRID>
+struct PatchShape64 {
+  static constexpr int a(int quad) { return quad == 1 || (GRID && (quad == 3 || quad == 7)) ? 1 : 2; }   // batches
+  static constexpr int off_a(int quad) { return quad == 0 ? 0 : off_bt(quad - 1) + (quad == 2 ? 0 : 128); }
+  static constexpr int off_bt(int quad) { return off_a(quad) + 128 * a(quad); }   // (none in quad 1)
+  static constexpr int own = off_bt(7) + 128;
+  static constexpr int words = own + 16;
+};
+
 struct PatchTables {
   bool ok = false;           // false: some patch does not fit, the two-launch form is used
   int stride = 0;            // ints per record
   int n_buffers = 1;         // copies of the velocity the step alternates between
   int n_patterns = 0;
-  bool grid = false;         // the patterns have PatchShape<true>, else PatchShape<false>
+  bool grid = false;         // the patterns have PatchShape*<true>, else <false>
   std::vector<int> rec;
   std::vector<uint32_t> pat;
 };
 
 // ug / pg: 27 velocity and 4 pressure dofs of every cell; cells of color k are
-// order[ptr[k] .. ptr[k + 1])
+// order[ptr[k] .. ptr[k + 1]); fp64: patterns of PatchShape64
 void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, const std::vector<int> &pg, int n_colors,
-                        const int *ptr, const int *order, PatchTables &out);
+                        const int *ptr, const int *order, bool fp64, PatchTables &out);
 
 }  // namespace pmg

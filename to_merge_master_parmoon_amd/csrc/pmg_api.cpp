@@ -663,7 +663,8 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   // size faster than the two launches (k_patch.hip); these stay for refinement steps, nine
   // blocks, stored LU factors and levels whose patches fit no record (rows of more than 128
   // entries, shared pressure dofs, colors that share dofs)
-  const bool fused = ua && D.patch_rec && nref == 0;
+  const bool fused = sizeof(T) == 8 ? rloc == reinterpret_cast<T *>(D.rloc) && D.patch_rec && D.a_shared
+                                    : ua && D.patch_rec && nref == 0;
   const bool full = !D.schur;
   for (int col = 0; col < D.n_colors; ++col) {
     const int p0 = D.ptr_colors[col];
@@ -695,6 +696,14 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
         launch_patch_step(P, D.minv32, D.minv16, full, c->stream);
         continue;
       }
+    } else if (fused) {
+      const double by = D.res_bytes[1][0][col] * part - nc * (31.0 * 20 + 85 * 8.0) +
+                        nc * (NLOC * NLOC * 8.0 + 4.0 * D.patch_stride + 85 * 8.0);
+      Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
+      PatchStep64 P{D.patch_rec, D.patch_pat, slots, D.invperm, op.a1, op.btv, op.bv, f, D.lu, u, D.patch_alt, damp,
+                    D.patch_stride, D.n_udof, nc, p0, nc >= XCD_GROUP_MIN && D.tune_res_xcd[0], D.patch_grid};
+      launch_patch_step64(P, c->stream);
+      continue;
     }
     {
       const double rb = D.res_bytes[D.a_shared][vs == 8 ? 0 : 1][col] * part;
@@ -2236,9 +2245,9 @@ static int add_level(pmg_ctx *c, const pmg_level_desc *d, int *level_out, bool m
         D.minv16 = dalloc<uint16_t>(c, minvn);
         launch_fill<uint16_t>(D.minv16, uint16_t(0), long(minvn), c->stream);
       }
-      if (D.minv32 || D.minv16) {
+      if (D.lu || D.minv32 || D.minv16) {
         PatchTables T;
-        build_patch_tables(d, ug, pg, nc, D.ptr_colors.data(), reo.data(), T);
+        build_patch_tables(d, ug, pg, nc, D.ptr_colors.data(), reo.data(), D.lu != nullptr, T);
         if (T.ok) {
           D.patch_rec = dalloc<int>(c, T.rec.size());
           h2d(c, D.patch_rec, T.rec.data(), T.rec.size());
@@ -2249,11 +2258,15 @@ static int add_level(pmg_ctx *c, const pmg_level_desc *d, int *level_out, bool m
           D.patch_grid = T.grid;
           PMG_HIP_CHECK(hipStreamSynchronize(c->stream));
         }
+      }
+      if (D.lu) {
+        if (D.patch_rec) D.patch_alt = dalloc<double>(c, 3 * size_t(D.n_udof) * std::max(1, D.patch_buffers - 1));
+      } else if (D.minv32 || D.minv16) {
         D.ua32 = dalloc<float>(c, 4 * size_t(D.n_udof) * D.patch_buffers);
       } else if (c->prm.precision == PMG_PREC_FP32) {
         D.lu32 = dalloc<float>(c, lun);
         launch_fill<float>(D.lu32, 0.0f, long(lun), c->stream);
-      } else {
+      } else if (c->prm.precision == PMG_PREC_FP32_BF16) {
         D.lu16 = dalloc<uint16_t>(c, lun);
         PMG_HIP_CHECK(hipMemsetAsync(D.lu16, 0, lun * sizeof(uint16_t), c->stream));
       }

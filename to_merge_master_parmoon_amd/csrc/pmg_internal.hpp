@@ -175,6 +175,7 @@ struct DevLevel {
   uint32_t *patch_pat = nullptr;
   int patch_stride = 0, patch_buffers = 1;
   bool patch_grid = false;
+  double *patch_alt = nullptr;       // FP64: the copies of the velocity after the first
   // the patch inverses are stored in the block form (set at every factorization: shared
   // velocity block present)
   bool schur = false;
@@ -396,6 +397,20 @@ struct PatchStep {
   int mirror;                 // 1: u takes the new velocity too
   int grid;                   // PatchShape<true>, else <false>
 };
+// the same of the FP64 sweep with the shared block and stored LU factors; alt: the copies of the
+// velocity after u itself, three component vectors of N each
+struct PatchStep64 {
+  const int *rec;
+  const uint32_t *pat;
+  const int *slots;
+  const uint8_t *invperm;
+  const double *a1, *btv, *bv, *f, *lu;
+  double *u, *alt;
+  double damp;
+  int stride, N, ncells, pos0;
+  int grouped, grid;
+};
+void launch_patch_step64(const PatchStep64 &P, hipStream_t s);
 // full: the stored data is the full inverse, else the block form
 void launch_patch_step(const PatchStep &P, const float *stored32, const uint16_t *stored16, bool full, hipStream_t s);
 template <typename T, typename F>
