@@ -29,6 +29,7 @@
 #include "pmg_internal.hpp"
 #include "pmg_rows.hpp"
 #include "coarse_rows.hpp"
+#include "wave_argmax.hpp"
 
 namespace pmg {
 
@@ -37,39 +38,6 @@ namespace {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 __device__ inline d4 mfma16(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-
-// (bv, bi) := the larger value, the lower index among equals (the pivot rule of dgetf2)
-__device__ inline void amax_take(double &bv, int &bi, double ov, int oi) {
-  const bool take = ov > bv || (ov == bv && oi < bi);
-  bv = take ? ov : bv;
-  bi = take ? oi : bi;
-}
-// one step of the reduction with the partner lane that the DPP pattern CTRL selects
-template <int CTRL>
-__device__ inline void amax_dpp(double &bv, int &bi) {
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(bv), CTRL, 0xF, 0xF, false);
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(bv), CTRL, 0xF, 0xF, false);
-  const int oi = __builtin_amdgcn_mov_dpp(bi, CTRL, 0xF, 0xF, false);
-  amax_take(bv, bi, __hiloint2double(hi, lo), oi);
-}
-// the wavefront's largest value and its lowest index in every lane (all 64 lanes active):
-// within each row of 16 lanes by DPP (quad xor 1, quad xor 2, half-row mirror, row
-// mirror), then the four rows' results by readlane, taken in lane order
-__device__ inline void wave_argmax(double &bv, int &bi) {
-  amax_dpp<0xB1>(bv, bi);
-  amax_dpp<0x4E>(bv, bi);
-  amax_dpp<0x141>(bv, bi);
-  amax_dpp<0x140>(bv, bi);
-  const int h = __double2hiint(bv), l = __double2loint(bv);
-  double v = __hiloint2double(__builtin_amdgcn_readlane(h, 0), __builtin_amdgcn_readlane(l, 0));
-  int i = __builtin_amdgcn_readlane(bi, 0);
-#pragma unroll
-  for (int r = 1; r < 4; ++r)
-    amax_take(v, i, __hiloint2double(__builtin_amdgcn_readlane(h, 16 * r), __builtin_amdgcn_readlane(l, 16 * r)),
-              __builtin_amdgcn_readlane(bi, 16 * r));
-  bv = v;
-  bi = i;
-}
 
 constexpr int LU_NB = 16;          // panel width
 constexpr int LU_T = 512;          // threads of the single-workgroup LU (one panel row each)
@@ -469,6 +437,137 @@ __global__ __launch_bounds__(TRSM_T) void k_trsm_wg(const double *__restrict__ l
   }
 }
 
+// The same for 512 < n <= TRSM_BIG_N: the slab takes the LDS that k_trsm_wg stages factor blocks
+// in, so the updates read their factor tiles from memory straight into the matrix cores'
+// operands, all tiles of a wavefront (8) in flight and issued before the diagonal solve.  Bound
+// by the chain of n / 16 blocks twice, two barriers and a diagonal solve each: n = 729 with 2226
+// right-hand sides (140 workgroups) 0.78 ms.
+constexpr int TRSM_BIG_N = 1024, TRSM_BIG_T = 512;
+// the loads through p after this come after the steps that x waits for (left alone, the compiler
+// loads the whole diagonal block first and spills)
+__device__ __forceinline__ void step_in_order(const double *&p, double (&x)[16]) {
+  int off = 0;
+  asm volatile("" : "+v"(off), "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]),
+                    "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]),
+                    "+v"(x[14]), "+v"(x[15]));
+  p += off;
+}
+__global__ __launch_bounds__(TRSM_BIG_T) void k_trsm_big(const double *__restrict__ lu, int n, int ld,
+                                                         const int *__restrict__ sigma, const double *__restrict__ R,
+                                                         int ldr, int nrhs, double *__restrict__ X, int ldx) {
+  constexpr int NW = TRSM_BIG_T / 64, TPW = TRSM_BIG_N / 16 / NW;   // wavefronts, tiles of one
+  __shared__ double xs[TRSM_BIG_N][TRSM_NR + 1];
+  __shared__ double dg[16][17];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int c0 = blockIdx.x * TRSM_NR;
+#pragma unroll 1
+  for (int idx = t; idx < n * TRSM_NR; idx += TRSM_BIG_T) {
+    const int i = idx / TRSM_NR, cc = idx - i * TRSM_NR, c = c0 + cc;
+    double v = 0.0;
+    if (c < nrhs) v = R ? R[long(sigma[i]) * ldr + c] : (sigma[i] == c ? 1.0 : 0.0);
+    xs[i][cc] = v;
+  }
+  const int nb = (n + 15) / 16;
+  const int col = lane & 15, rq = lane >> 4;
+  double av[TPW][4];
+  // factor tiles (rows of block tb, columns of block kb) of this wavefront: tb = first + wave + NW j
+  auto fetch = [&](int first, int end, int k0, int kw) {
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) {
+      const int tb = first + wave + NW * j, i = tb * 16 + col;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool in = tb < end && i < n && 4 * s + rq < kw;
+        const double v = lu[in ? long(i) * ld + k0 + 4 * s + rq : 0];
+        av[j][s] = in ? -v : 0.0;
+      }
+    }
+  };
+  auto update = [&](int first, int end, int k0, int kw) {
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) {
+      const int tb = first + wave + NW * j;
+      if (tb >= end) continue;
+      d4 acc;
+#pragma unroll
+      for (int qq = 0; qq < 4; ++qq) {
+        const int i = tb * 16 + 4 * qq + rq;
+        acc[qq] = i < n ? xs[i][col] : 0.0;
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = mfma16(av[j][s], 4 * s + rq < kw ? xs[k0 + 4 * s + rq][col] : 0.0, acc);
+#pragma unroll
+      for (int qq = 0; qq < 4; ++qq) {
+        const int i = tb * 16 + 4 * qq + rq;
+        if (i < n) xs[i][col] = acc[qq];
+      }
+    }
+  };
+  // forward: unit lower L
+#pragma unroll 1
+  for (int kb = 0; kb < nb; ++kb) {
+    const int k0 = kb * 16, kw = min(16, n - k0);
+    fetch(kb + 1, nb, k0, kw);
+    if (t < 256) {
+      const int i = t >> 4, k = t & 15;
+      dg[i][k] = (i < kw && k < kw) ? lu[long(k0 + i) * ld + k0 + k] : 0.0;
+    }
+    __syncthreads();
+    if (t < TRSM_NR) {
+      double x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = i < kw ? xs[k0 + i][t] : 0.0;
+      const double *d = &dg[0][0];
+#pragma unroll
+      for (int k = 0; k < 15; ++k) {
+        step_in_order(d, x);
+#pragma unroll
+        for (int i = k + 1; i < 16; ++i) x[i] = fma(-d[17 * i + k], x[k], x[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (i < kw) xs[k0 + i][t] = x[i];
+    }
+    __syncthreads();
+    update(kb + 1, nb, k0, kw);
+  }
+  // backward: upper U with its diagonal
+#pragma unroll 1
+  for (int kb = nb - 1; kb >= 0; --kb) {
+    const int k0 = kb * 16, kw = min(16, n - k0);
+    fetch(0, kb, k0, kw);
+    if (t < 256) {
+      const int i = t >> 4, k = t & 15;
+      dg[i][k] = (i < kw && k < kw) ? lu[long(k0 + i) * ld + k0 + k] : 1.0;
+    }
+    __syncthreads();
+    if (t < TRSM_NR) {
+      double x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = i < kw ? xs[k0 + i][t] : 0.0;
+      const double *d = &dg[0][0];
+#pragma unroll
+      for (int k = 15; k >= 0; --k) {
+        step_in_order(d, x);
+        x[k] = x[k] / d[18 * k];
+#pragma unroll
+        for (int i = 0; i < k; ++i) x[i] = fma(-d[17 * i + k], x[k], x[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (i < kw) xs[k0 + i][t] = x[i];
+    }
+    __syncthreads();
+    update(0, kb, k0, kw);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int idx = t; idx < n * TRSM_NR; idx += TRSM_BIG_T) {
+    const int i = idx / TRSM_NR, cc = idx - i * TRSM_NR, c = c0 + cc;
+    if (c < nrhs) X[long(i) * ldx + c] = xs[i][cc];
+  }
+}
+
 // ------------------------------------------------------------------ FP64 GEMM
 // C = alpha A B + beta C (row-major; A M x K, B K x N); one wavefront per 16 x 16 tile of C,
 // four per workgroup, K in steps of 4 on the matrix cores.
@@ -565,7 +664,12 @@ __global__ __launch_bounds__(256) void k_cbb_phase2(const CbJob *__restrict__ jo
 
 }  // namespace
 
-bool coarse_block_fits(int m, int q) { return m > 0 && q > 0 && m <= LU_T && q <= LU_T; }
+// A up to 512 unknowns is factored by one workgroup, up to 1024 (a 5^3 grid with three natural
+// faces has 1000) by the panel launches of the whole system's LU; beyond that the slab of
+// k_trsm_big exceeds LDS.  5^3 (729 + 499): set-up about 15 -> 6.5 ms, a visit 630 -> 33 us against the
+// LU of the 2686 unknowns.
+bool coarse_block_fits(int m, int q) { return m > 0 && q > 0 && m <= TRSM_BIG_N && q <= LU_T; }
+bool coarse_block_panels(int m) { return m > LU_T; }
 
 void launch_cb_build(const DevLevel &L, CoarseBlock &B, hipStream_t s) {
   const long m = B.m, q = B.q;
@@ -594,9 +698,15 @@ void coarse_block_factor(CoarseBlock &B, hipStream_t s) {
   const int ldx = m + 3 * q;          // X = [Ainv | W1 W2 W3]
   const int ldp = 3 * m + q;          // P1 = [-Q1 -Q2 -Q3 | S^{-1}]
   // A = P^T L U; X = A^{-1} [I | BT1 BT2 BT3] (in place: the solve reads its slab first)
-  k_lu_wg<<<1, LU_T, 0, s>>>(B.A, m, m, B.sigA, B.info);
-  PMG_HIP_CHECK(hipGetLastError());
-  k_trsm_wg<<<(ldx + TRSM_NR - 1) / TRSM_NR, TRSM_T, 0, s>>>(B.A, m, m, B.sigA, B.X, ldx, ldx, B.X, ldx);
+  const int slabs = (ldx + TRSM_NR - 1) / TRSM_NR;
+  if (coarse_block_panels(m)) {
+    lu_factor_panels(B.A, m, B.ipiv, B.sigA, B.ubuf, B.swp, B.info, s);
+    k_trsm_big<<<slabs, TRSM_BIG_T, 0, s>>>(B.A, m, m, B.sigA, B.X, ldx, ldx, B.X, ldx);
+  } else {
+    k_lu_wg<<<1, LU_T, 0, s>>>(B.A, m, m, B.sigA, B.info);
+    PMG_HIP_CHECK(hipGetLastError());
+    k_trsm_wg<<<slabs, TRSM_T, 0, s>>>(B.A, m, m, B.sigA, B.X, ldx, ldx, B.X, ldx);
+  }
   PMG_HIP_CHECK(hipGetLastError());
   // S = -sum_b B_b W_b
   for (int b = 0; b < 3; ++b)

@@ -14,6 +14,7 @@
 // order); each visit runs blocked column sweeps in the dgetrs order.
 #include "pmg_internal.hpp"
 #include "pmg_rows.hpp"
+#include "wave_argmax.hpp"
 #include "coarse_rows.hpp"
 
 namespace pmg {
@@ -116,30 +117,24 @@ __global__ __launch_bounds__(PT) void k_lu_panel(double *__restrict__ a, int n, 
           }
         }
       }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(bv, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (ov > bv || (ov == bv && oi < bi)) {
-          bv = ov;
-          bi = oi;
-        }
-      }
+      wave_argmax(bv, bi);
       if (lane == 0) {
         sv[par][wave] = bv;
         si[par][wave] = bi;
       }
       __syncthreads();
-      bv = sv[par][0];
-      bi = si[par][0];
+      {
+        double cv[PT / 64];
+        int ci[PT / 64];
 #pragma unroll
-      for (int w2 = 1; w2 < PT / 64; ++w2) {
-        const double ov = sv[par][w2];
-        const int oi = si[par][w2];
-        if (ov > bv || (ov == bv && oi < bi)) {
-          bv = ov;
-          bi = oi;
+        for (int w2 = 0; w2 < PT / 64; ++w2) {
+          cv[w2] = sv[par][w2];
+          ci[w2] = si[par][w2];
         }
+        bv = cv[0];
+        bi = ci[0];
+#pragma unroll
+        for (int w2 = 1; w2 < PT / 64; ++w2) amax_take(bv, bi, cv[w2], ci[w2]);
       }
       const int p = bi;
       const bool nz = bv != 0.0;
@@ -575,12 +570,10 @@ void launch_coarse_build(const DevLevel &L, Coarse &C, hipStream_t s) {
   const int rows = L.n_udof + L.n_pdof;
   k_coarse_scatter<<<(rows * 16 + 255) / 256, 256, 0, s>>>(L.op64(), C.a, n, C.pin);
   PMG_HIP_CHECK(hipGetLastError());
-  k_iota<<<int((n + 255) / 256), 256, 0, s>>>(C.sigma, int(n));
-  PMG_HIP_CHECK(hipGetLastError());
 }
 
-void coarse_lu_factor(Coarse &C, hipStream_t s) {
-  const int n = C.n;
+// a (n x n, row-major) := L U by panels, sigma[i] = original row now at row i
+void lu_factor_panels(double *a, int n, int *ipiv, int *sigma, double *ubuf, int *swp, int *info, hipStream_t s) {
   const int pr_max = 7;   // PR = 7 spills 16 VGPRs to scratch; 8 would spill ~1000
   if ((n + PNT - 1) / PNT > pr_max)
     throw DeviceError("coarse system of " + std::to_string(n) + " unknowns exceeds the dense LU limit (" +
@@ -588,13 +581,15 @@ void coarse_lu_factor(Coarse &C, hipStream_t s) {
   // panels of 256 threads while they fit (measured faster: 6.7 vs 6.9 ms for the 1284
   // system beside the patch set-up), 512 above
   const bool narrow = (n + 255) / 256 <= pr_max;
-  PMG_HIP_CHECK(hipMemsetAsync(C.info, 0, sizeof(int), s));
+  PMG_HIP_CHECK(hipMemsetAsync(info, 0, sizeof(int), s));
+  k_iota<<<(n + 255) / 256, 256, 0, s>>>(sigma, n);
+  PMG_HIP_CHECK(hipGetLastError());
   int pj0 = 0, pj1 = 0;
   for (int j0 = 0; j0 < n; j0 += NBR) {
     const int j1 = std::min(n, j0 + NBR);
     const int pt = narrow ? 256 : PNT;
     const int pr = (n - j0 + pt - 1) / pt;
-#define PMG_PANEL(P, T) k_lu_panel<P, T><<<1, T, 0, s>>>(C.a, n, j0, j1, C.ipiv, C.info, C.swp, C.sigma)
+#define PMG_PANEL(P, T) k_lu_panel<P, T><<<1, T, 0, s>>>(a, n, j0, j1, ipiv, info, swp, sigma)
     if (narrow) {
       switch (pr) {
         case 1: PMG_PANEL(1, 256); break;
@@ -618,11 +613,11 @@ void coarse_lu_factor(Coarse &C, hipStream_t s) {
     }
 #undef PMG_PANEL
     PMG_HIP_CHECK(hipGetLastError());
-    k_lu_swap<<<(n + 255) / 256, 256, 0, s>>>(C.a, n, j0, j1, C.swp, C.ubuf, pj0, pj1);
+    k_lu_swap<<<(n + 255) / 256, 256, 0, s>>>(a, n, j0, j1, swp, ubuf, pj0, pj1);
     PMG_HIP_CHECK(hipGetLastError());
     if (j1 < n) {
       dim3 g((n - j1 + 63) / 64, (n - j1 + 63) / 64);
-      k_lu_update<<<g, 256, 0, s>>>(C.a, C.ubuf, n, j0, j1);
+      k_lu_update<<<g, 256, 0, s>>>(a, ubuf, n, j0, j1);
       PMG_HIP_CHECK(hipGetLastError());
       pj0 = j0;
       pj1 = j1;
@@ -630,6 +625,11 @@ void coarse_lu_factor(Coarse &C, hipStream_t s) {
       pj0 = pj1 = 0;
     }
   }
+}
+
+void coarse_lu_factor(Coarse &C, hipStream_t s) {
+  const int n = C.n;
+  lu_factor_panels(C.a, n, C.ipiv, C.sigma, C.ubuf, C.swp, C.info, s);
   dim3 gt((n + 63) / 64, (n + 63) / 64);
   k_transpose<<<gt, 256, 0, s>>>(C.a, C.f, n);
   PMG_HIP_CHECK(hipGetLastError());

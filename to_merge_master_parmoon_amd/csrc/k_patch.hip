@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256) void k_patch_step(PatchStep P, const F *__rest
 // Bounds: small colors the chain of 170 steps of the two sweeps (lu_sweeps.hpp); large ones the
 // stream of factors and rows, 100 KB per patch (226 registers allow two workgroups per CU, whose
 // loads in flight cover the latency).  Residual and solve launches before -> this one, per color:
-// 8^3 5.8 + 9.5 -> 9.2 us, 16^3 11.5 + 13.8 -> 15.8 us, 12 x 16 x 20 10.9 + 13.2 -> 14.8 us; the
+// 8^3 5.8 + 9.5 -> 9.2 us, 16^3 11.5 + 13.8 -> 15.8 us, 12 x 16 x 20 10.9 + 13.2 -> 15.9 us; the
 // set-up and solve at 32^3 72.0 -> 54.7 ms.  The same results bit for bit.
 __device__ __forceinline__ double *velocity_at(const PatchStep64 &P, int loc) {
   double *p = P.u + loc;

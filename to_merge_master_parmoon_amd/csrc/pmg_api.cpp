@@ -1109,9 +1109,12 @@ void coarse_alloc(pmg_ctx *c, Coarse &C, int nr) {
 void coarse_block_alloc(pmg_ctx *c, CoarseBlock &B, int m, int q) {
   if (B.A && (B.m != m || B.q != q)) {
     for (void *p : {(void *)B.A, (void *)B.X, (void *)B.B, (void *)B.V, (void *)B.S, (void *)B.P1, (void *)B.rr,
-                    (void *)B.y, (void *)B.p, (void *)B.sigA, (void *)B.sigS, (void *)B.iota})
+                    (void *)B.y, (void *)B.p, (void *)B.sigA, (void *)B.sigS, (void *)B.iota, (void *)B.ipiv,
+                    (void *)B.swp, (void *)B.ubuf})
       dfree(c, p);
     B.A = nullptr;
+    B.ipiv = B.swp = nullptr;
+    B.ubuf = nullptr;
   }
   if (B.A) return;
   B.m = m;
@@ -1129,6 +1132,11 @@ void coarse_block_alloc(pmg_ctx *c, CoarseBlock &B, int m, int q) {
   B.sigA = dalloc<int>(c, M);
   B.sigS = dalloc<int>(c, Q);
   B.iota = dalloc<int>(c, 3 * M + Q);
+  if (coarse_block_panels(m)) {
+    B.ipiv = dalloc<int>(c, M);
+    B.swp = dalloc<int>(c, 4 * 16 + 1);
+    B.ubuf = dalloc<double>(c, M * 16);
+  }
   std::vector<int> id(3 * M + Q);
   std::iota(id.begin(), id.end(), 0);
   h2d(c, B.iota, id.data(), id.size());

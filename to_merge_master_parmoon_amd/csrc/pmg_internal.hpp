@@ -288,6 +288,9 @@ struct CoarseBlock {
   double *A = nullptr, *X = nullptr, *B = nullptr, *V = nullptr, *S = nullptr, *P1 = nullptr;
   double *rr = nullptr, *y = nullptr, *p = nullptr;
   int *sigA = nullptr, *sigS = nullptr, *iota = nullptr, *info = nullptr;
+  // (coarse_block_panels) work arrays of the panel LU, as in Coarse
+  int *ipiv = nullptr, *swp = nullptr;
+  double *ubuf = nullptr;
 };
 
 // Coarse level: the dense system of SolveExact with the Dirichlet rows (identity) and the
@@ -460,6 +463,8 @@ void launch_coarse_rhs(const OpView<double> &op, const double *f, const int *sig
 // (asynchronous; cb.info gets the zero-pivot flags of the two LUs) and one visit from the
 // reduced right-hand side rr into the level vector u
 bool coarse_block_fits(int m, int q);
+bool coarse_block_panels(int m);   // A is factored by lu_factor_panels (info[0] gets its zero-pivot flag)
+void lu_factor_panels(double *a, int n, int *ipiv, int *sigma, double *ubuf, int *swp, int *info, hipStream_t s);
 void launch_cb_build(const DevLevel &L, CoarseBlock &B, hipStream_t s);
 void coarse_block_factor(CoarseBlock &B, hipStream_t s);
 void coarse_block_solve(CoarseBlock &B, const OpView<double> &op, const double *rr, const double *f, double *u,
