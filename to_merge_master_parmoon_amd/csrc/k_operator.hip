@@ -6,9 +6,8 @@
 // contiguous 16-entry segments; the three velocity components of a row are produced
 // together so x is gathered once per entry.  Pressure rows follow the velocity rows in
 // the same launch.  Reductions that the reference performs after the product (IntoL20
-// mean of the P1disc constants, the Euclidean norm) are folded into the same launch with a
-// deterministic last-block finish: every block writes its partial sums, the block that
-// arrives last sums them in a fixed order and applies the projection.
+// mean of the P1disc constants, the Euclidean norm) are partial sums per block, added up in a
+// fixed order by small launches that follow.
 #include "pmg_internal.hpp"
 #include "pmg_rows.hpp"
 
@@ -37,41 +36,22 @@ __device__ inline void block_sum2(double &a, double &b, double *sh) {
   b = (sh[4] + sh[5]) + (sh[6] + sh[7]);
 }
 
-// Last block of the grid sums partials[0..nblk) (two values each) in a fixed order.
-// Returns true in every thread of the last block.
-__device__ inline bool last_block_sum2(double pa, double pb, double *partials, unsigned *counter,
-                                       double &ta, double &tb, double *sh) {
-  __shared__ bool am_last;
+// this block's two sums into partials[2 block], added up by k_sum2 in a second launch (a
+// last-block finish costs every block a fence and an atomic on one counter: the 32^3 defect
+// with its norm 379 us instead of 195)
+__device__ inline void put_partials2(double pa, double pb, double *partials, double *sh) {
   block_sum2(pa, pb, sh);
   if (threadIdx.x == 0) {
     partials[2 * blockIdx.x] = pa;
     partials[2 * blockIdx.x + 1] = pb;
-    __threadfence();
-    unsigned prev = atomicAdd(counter, 1u);
-    am_last = (prev == gridDim.x - 1);
   }
-  __syncthreads();
-  if (!am_last) return false;
-  __threadfence();
-  double a = 0, b = 0;
-  for (int i = threadIdx.x; i < int(gridDim.x); i += 256) {
-    a += static_cast<volatile double *>(partials)[2 * i];
-    b += static_cast<volatile double *>(partials)[2 * i + 1];
-  }
-  __syncthreads();
-  block_sum2(a, b, sh);
-  ta = a;
-  tb = b;
-  if (threadIdx.x == 0) *counter = 0u;
-  return true;
 }
 
 // SH: the velocity coupling is the shared block op.a1 (one value stream instead of nine)
 template <int MODE, typename T, bool SH>
 __global__ __launch_bounds__(256) void k_type4(OpView<T> op, const T *__restrict__ x,
                                                const T *__restrict__ bv, T *__restrict__ y,
-                                               int project, int want_norm, double *partials,
-                                               unsigned *counter, double *res, double *res_slots) {
+                                               int project, int want_norm, double *partials) {
   __shared__ double sh[8];
   const int lane = threadIdx.x & 15, grp = threadIdx.x >> 4;
   const int N = op.n_udof, NA = op.n_active, NP = op.n_pdof;
@@ -144,25 +124,33 @@ __global__ __launch_bounds__(256) void k_type4(OpView<T> op, const T *__restrict
       }
     }
   }
-  if (!(project || want_norm)) return;
-  double tpc, tsq;
-  if (!last_block_sum2(pc, sq, partials, counter, tpc, tsq, sh)) return;
-  if (threadIdx.x == 0) {
-    if (project) {
-      // IntoL20Vector3D case -11 (MGComponents3D.C:1766-1786): s = sum/Length*4, applied by
-      // k_l20_apply; the squares of the constants are added there
-      res_slots[0] = tpc / double(NP) * 4.0;
-      res_slots[1] = tsq;
-    } else {
-      *res = sqrt(tsq);
-    }
+  if (project || want_norm) put_partials2(pc, sq, partials, sh);
+}
+
+// the sums of np block partials in a fixed order: with NP > 0 slots = {mean of the P1disc
+// constants (IntoL20Vector3D case -11, MGComponents3D.C:1766-1786: sum / Length * 4), the squares
+// of the rest} for k_l20_apply, else *res = sqrt(base + squares)
+__global__ __launch_bounds__(256) void k_sum2(const double *__restrict__ partials, int np, int NP, double *slots,
+                                              const double *base, double *res) {
+  __shared__ double sh[8];
+  double a = 0, b = 0;
+  for (int i = threadIdx.x; i < np; i += 256) {
+    a += partials[2 * i];
+    b += partials[2 * i + 1];
+  }
+  block_sum2(a, b, sh);
+  if (threadIdx.x != 0) return;
+  if (NP > 0) {
+    slots[0] = a / double(NP) * 4.0;
+    slots[1] = b;
+  } else {
+    *res = sqrt((base ? *base : 0.0) + b);
   }
 }
 
-// v[4i] -= s for the P1disc constants; with res: ||.||^2 = base + sum of the new squares
+// v[4i] -= slots[0] for the P1disc constants; partials (may be null): the sums of the new squares
 template <typename T>
-__global__ __launch_bounds__(256) void k_l20_apply(T *__restrict__ p, int NP, const double *slots, double *res,
-                                                   double *partials, unsigned *counter) {
+__global__ __launch_bounds__(256) void k_l20_apply(T *__restrict__ p, int NP, const double *slots, double *partials) {
   __shared__ double sh[8];
   const double m = slots[0];
   double add = 0.0;
@@ -171,9 +159,7 @@ __global__ __launch_bounds__(256) void k_l20_apply(T *__restrict__ p, int NP, co
     p[4 * i] = v;
     add += double(v) * v;
   }
-  if (!res) return;
-  double t, u;
-  if (last_block_sum2(add, 0.0, partials, counter, t, u, sh) && threadIdx.x == 0) *res = sqrt(slots[1] + t);
+  if (partials) put_partials2(0.0, add, partials, sh);
 }
 
 template <typename T>
@@ -373,46 +359,46 @@ void launch_type4(const OpView<T> &op, int mode, const T *x, const T *b, T *y, b
   if (op.rows && (want_norm || proj))
     throw DeviceError("launch_type4: a row subset is supported without the norm and the projection only");
   if (n_rows <= 0) return;
-  const int grid = chunk_grid(n_rows, op.rpb > 0 ? op.rpb : 64, RED_BLOCKS);
-  auto go = [&](auto mode_c, int pr, int wn, double *rs, double *sl) {
+  // rows per workgroup where the autotuner set none: 64 (four per 16-lane group, one after the
+  // other) once that gives 2048 workgroups, down to one per group on smaller levels, which are
+  // bound by that chain (FP32 defect at 8^3 13.0 -> 5.0 us, 12^3 15.2 -> 7.3, 16^3 18.8 -> 13.3)
+  const int auto_rpb = int(std::min(64L, std::max(16L, n_rows / 2048 / 16 * 16)));
+  const int grid = chunk_grid(n_rows, op.rpb > 0 ? op.rpb : auto_rpb, RED_BLOCKS);
+  auto go = [&](auto mode_c, int pr, int wn) {
     constexpr int M = decltype(mode_c)::value;
     if (op.a1)
-      k_type4<M, T, true><<<grid, 256, 0, s>>>(op, x, b, y, pr, wn, red.partials, red.counter, rs, sl);
+      k_type4<M, T, true><<<grid, 256, 0, s>>>(op, x, b, y, pr, wn, red.partials);
     else
-      k_type4<M, T, false><<<grid, 256, 0, s>>>(op, x, b, y, pr, wn, red.partials, red.counter, rs, sl);
+      k_type4<M, T, false><<<grid, 256, 0, s>>>(op, x, b, y, pr, wn, red.partials);
+    PMG_HIP_CHECK(hipGetLastError());
   };
   using M0 = std::integral_constant<int, 0>;
   using M1 = std::integral_constant<int, 1>;
   using M2 = std::integral_constant<int, 2>;
-  if (proj && !want_norm) {
-    // the product without a grid-wide reduction (no per-block fence and counter atomic),
-    // then the projection in two small passes
-    if (mode == 1)
-      go(M1{}, 0, 0, nullptr, nullptr);
-    else
-      go(M2{}, 0, 0, nullptr, nullptr);
-    PMG_HIP_CHECK(hipGetLastError());
-    const int g = std::max(1, std::min(64, op.n_pdof / 4 / 2048));
-    k_l20_part<T><<<g, 256, 0, s>>>(y + 3L * op.n_udof, op.n_pdof, red.partials);
-    k_l20_sub<T><<<g, 256, 0, s>>>(y + 3L * op.n_udof, op.n_pdof, red.partials);
-    PMG_HIP_CHECK(hipGetLastError());
-    return;
-  }
-  double *slots = red.result + 8;
+  const bool in_launch = proj && want_norm;   // with the norm, the constants are summed in the product
   if (mode == 0)
-    go(M0{}, 0, want_norm, res, slots);
+    go(M0{}, 0, want_norm);
   else if (mode == 1)
-    go(M1{}, proj, want_norm, res, slots);
+    go(M1{}, in_launch, want_norm);
   else
-    go(M2{}, proj, want_norm, res, slots);
-  PMG_HIP_CHECK(hipGetLastError());
-  if (proj) {
-    const int nc = op.n_pdof / 4;
-    const int g = std::max(1, std::min(512, (nc + 255) / 256));
-    k_l20_apply<T><<<g, 256, 0, s>>>(y + 3L * op.n_udof, op.n_pdof, slots, want_norm ? res : nullptr,
-                                     red.partials, red.counter);
-    PMG_HIP_CHECK(hipGetLastError());
+    go(M2{}, in_launch, want_norm);
+  T *const p = y + 3L * op.n_udof;
+  if (proj && !want_norm) {
+    // the projection in two small passes
+    const int g = std::max(1, std::min(64, op.n_pdof / 4 / 2048));
+    k_l20_part<T><<<g, 256, 0, s>>>(p, op.n_pdof, red.partials);
+    k_l20_sub<T><<<g, 256, 0, s>>>(p, op.n_pdof, red.partials);
+  } else if (want_norm) {
+    double *slots = red.result + 8;
+    k_sum2<<<1, 256, 0, s>>>(red.partials, grid, proj ? op.n_pdof : 0, slots, nullptr, res);
+    if (proj) {
+      const int nc = op.n_pdof / 4;
+      const int g = std::max(1, std::min(512, (nc + 255) / 256));
+      k_l20_apply<T><<<g, 256, 0, s>>>(p, op.n_pdof, slots, red.partials);
+      k_sum2<<<1, 256, 0, s>>>(red.partials, g, 0, nullptr, slots + 1, res);
+    }
   }
+  PMG_HIP_CHECK(hipGetLastError());
 }
 template void launch_type4<double>(const OpView<double> &, int, const double *, const double *, double *, bool,
                                    double *, RedScratch &, hipStream_t);

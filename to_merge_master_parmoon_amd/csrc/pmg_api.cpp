@@ -455,6 +455,7 @@ void check_coarse(pmg_ctx *c, Coarse &C) {
 // row-blocked FP64 (and FP32) copies and, when the A blocks have it, the shared velocity
 // block form (FP64: block 0 of D.a read in place; FP32: its own copy)
 void drop_graph(pmg_ctx *c);
+void ensure_xa(pmg_ctx *c);
 
 void refresh_values(pmg_ctx *c, DevLevel &D) {
   launch_row_blocked<double>(D, D.av64, D.bv64, D.btv64, c->stream);
@@ -758,11 +759,37 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   }
 }
 
+// the buffer of the FP64 operator's interleaved input velocity, for the largest level
+void ensure_xa(pmg_ctx *c) {
+  long n = 0;
+  for (const auto &D : c->L) n = std::max<long>(n, D.n_udof);
+  if (c->batch || c->xa64_n >= n) return;
+  drop_graph(c);   // a captured V-cycle may hold the old buffer
+  dfree(c, c->xa64);
+  c->xa64 = nullptr;
+  c->xa64_n = 0;
+  c->xa64 = dalloc<double>(c, 4 * size_t(n));
+  c->xa64_n = n;
+}
+// With the shared velocity block the FP64 operator gathers an interleaved copy of its input's
+// velocity where that pays for the pass that makes it (3 x 8 B read, 4 x 8 B written per dof):
+// pmg_defect at 32^3 (274,625 velocity dofs) 198 -> 188 us, at 24^3 (117,649) 89 -> 90 us
+constexpr int XA_MIN_UDOF = 150000;
+OpView<double> op64_for(pmg_ctx *c, const DevLevel &D, const double *x) {
+  OpView<double> o = D.op64();
+  if (D.a_shared && c->xa64_n >= D.n_udof && D.n_udof >= XA_MIN_UDOF) {
+    launch_interleave3(c->xa64, x, D.n_udof, c->stream);
+    o.xa = c->xa64;
+  }
+  return o;
+}
+OpView<float> op64_for(pmg_ctx *, const DevLevel &D, const float *) { return D.op32(); }
+
 // res_dev (single problem only): ||d||_2 after the projection
 template <typename T>
 void mg_defect(pmg_ctx *c, const DevLevel &D, const T *u, const T *f, T *d, double *res_dev) {
   Timed tm(c, &c->tm.defect, D.defect_bytes[D.a_shared][sizeof(T) == 8 ? 0 : 1], 0.0);
-  launch_type4<T>(opview<T>(D), 2, u, f, d, fused_l20(c), c->batch ? nullptr : res_dev, c->red, c->stream);
+  launch_type4<T>(op64_for(c, D, u), 2, u, f, d, fused_l20(c), c->batch ? nullptr : res_dev, c->red, c->stream);
   if (c->batch) project_pressure<T>(c, D, d);
 }
 
@@ -1184,6 +1211,7 @@ void start_coarse_factor(pmg_ctx *c, const DevLevel &D, Coarse &C, int pin) {
 
 void setup_factors(pmg_ctx *c) {
   check_deferred(c);
+  ensure_xa(c);
   auto t0 = std::chrono::steady_clock::now();
   std::vector<Coarse *> todo;
   std::vector<const DevLevel *> todo_lvl;
@@ -1268,11 +1296,7 @@ void setup_factors(pmg_ctx *c) {
 }
 
 void ensure_fgmres(pmg_ctx *c) {
-  if (!c->batch && c->xa64_n != c->L.back().n_udof) {
-    dfree(c, c->xa64);
-    c->xa64_n = c->L.back().n_udof;
-    c->xa64 = dalloc<double>(c, 4 * size_t(c->xa64_n));
-  }
+  ensure_xa(c);
   const int m = std::max(1, std::min(c->prm.sc_gmres_restart > 0 ? c->prm.sc_gmres_restart : 10,
                                      std::max(1, c->prm.sc_lin_maxit_saddle)));
   if (m <= c->restart_alloc) return;
@@ -1311,7 +1335,7 @@ double dev_norm2(pmg_ctx *c, const double *x, long n) {
 void defect_nse4_dev(pmg_ctx *c, const double *x, const double *b, double *r) {
   DevLevel &F = c->L.back();
   Timed tm(c, &c->tm.matvec, F.defect_bytes[F.a_shared][0], 0.0);
-  launch_type4<double>(F.op64(), 1, x, b, r, fused_l20(c), nullptr, c->red, c->stream);
+  launch_type4<double>(op64_for(c, F, x), 1, x, b, r, fused_l20(c), nullptr, c->red, c->stream);
   if (c->batch) project_pressure<double>(c, F, r);
 }
 
@@ -1388,16 +1412,8 @@ int fgmres_dev(pmg_ctx *c, double *sol, const double *rhs, int *iters, double *f
     for (int i = 0; i < restart && j <= maxite; i++, j++) {
       for (int k = 0; k < std::max(1, P.sc_amg_prec_it); ++k) vcycle_dev(c, v(i), z(i));
       {
-        // with the shared velocity block the operator gathers an interleaved copy of the
-        // input's velocity (one pass more: 3 x 8 B read, 4 x 8 B written per velocity dof)
-        OpView<double> o = F.op64();
-        const bool il = F.a_shared && c->xa64;
-        Timed tm(c, &c->tm.matvec, F.matvec_bytes[F.a_shared] + (il ? 56.0 * F.n_udof : 0.0), 0.0);
-        if (il) {
-          launch_interleave3(c->xa64, z(i), F.n_udof, c->stream);
-          o.xa = c->xa64;
-        }
-        launch_type4<double>(o, 0, z(i), nullptr, c->W, false, nullptr, c->red, c->stream);
+        Timed tm(c, &c->tm.matvec, F.matvec_bytes[F.a_shared], 0.0);
+        launch_type4<double>(op64_for(c, F, z(i)), 0, z(i), nullptr, c->W, false, nullptr, c->red, c->stream);
       }
       // modified Gram-Schmidt, H[k][i] -> Hdev[k], ||w||^2 -> Hdev[i+1]
       launch_dot(c->W, v(0), n, c->Hdev, c->red, c->stream);
@@ -1935,9 +1951,7 @@ int pmg_ctx_create(int device, const pmg_params *params, pmg_ctx **out) {
     PMG_HIP_CHECK(hipEventCreate(&c->ev0));
     PMG_HIP_CHECK(hipEventCreate(&c->ev1));
     c->red.partials = dalloc<double>(c.get(), 2 * RED_BLOCKS + 16);
-    c->red.counter = dalloc<unsigned>(c.get(), 16);
     c->red.result = dalloc<double>(c.get(), 16);
-    PMG_HIP_CHECK(hipMemsetAsync(c->red.counter, 0, 16 * sizeof(unsigned), c->stream));
     PMG_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&c->hpin), sizeof(double) * 256));
     c->hpin_len = 256;
     PMG_HIP_CHECK(hipStreamSynchronize(c->stream));
@@ -2388,6 +2402,7 @@ int pmg_defect(pmg_ctx *c, int level, const double *u, const double *f, double *
     DevLevel &D = level_of(c, level);
     HostIO io(c, mem, D.n_dof);
     double *du = io.in(0, u), *df = io.in(1, f), *dd = (mem == PMG_MEM_HOST) ? c->stage[2] : d;
+    ensure_xa(c);
     mg_defect<double>(c, D, du, df, dd, c->red.result);
     if (c->batch) launch_dot(dd, dd, D.n_dof, c->red.result, c->red, c->stream);
     io.out(2, d);
@@ -2403,7 +2418,8 @@ int pmg_matvec(pmg_ctx *c, int level, const double *x, double *y, int mem) {
     DevLevel &D = level_of(c, level);
     HostIO io(c, mem, D.n_dof);
     double *dx = io.in(0, x), *dy = (mem == PMG_MEM_HOST) ? c->stage[2] : y;
-    launch_type4<double>(D.op64(), 0, dx, nullptr, dy, false, nullptr, c->red, c->stream);
+    ensure_xa(c);
+    launch_type4<double>(op64_for(c, D, dx), 0, dx, nullptr, dy, false, nullptr, c->red, c->stream);
     io.out(2, y);
     io.sync();
   });
@@ -2415,7 +2431,8 @@ int pmg_defect_nse4(pmg_ctx *c, int level, const double *x, const double *b, dou
     DevLevel &D = level_of(c, level);
     HostIO io(c, mem, D.n_dof);
     double *dx = io.in(0, x), *db = io.in(1, b), *dr = (mem == PMG_MEM_HOST) ? c->stage[2] : r;
-    launch_type4<double>(D.op64(), 1, dx, db, dr, fused_l20(c), nullptr, c->red, c->stream);
+    ensure_xa(c);
+    launch_type4<double>(op64_for(c, D, dx), 1, dx, db, dr, fused_l20(c), nullptr, c->red, c->stream);
     if (c->batch) project_pressure<double>(c, D, dr);
     io.out(2, r);
     io.sync();

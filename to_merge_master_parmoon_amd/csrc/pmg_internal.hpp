@@ -40,7 +40,7 @@ static_assert(SCH_END <= SCH_STRIDE && SCH_STRIDE <= MINV_STRIDE, "block-form pa
 constexpr int RLOC_STRIDE = 96;     // local residual slot (85 used)
 constexpr int POS_DOFS_STRIDE = 32; // dofs of the patch at a color position (27 + 4 used)
 constexpr int PERM_STRIDE = 96;     // uint8 inverse row permutation per patch
-constexpr int RED_BLOCKS = 4096;    // max blocks of the kernels with a last-block reduction
+constexpr int RED_BLOCKS = 4096;    // max blocks of the kernels with partial sums
 constexpr int ROW_PAD = 64;         // zeroed tail entries of the streamed operator arrays
 // per-cell gather map of the patch matrix (ints): offsets of the A entries (j, m) into the
 // row-blocked A values (block 0; -1: no entry), row lengths of the 27 velocity rows
@@ -323,10 +323,9 @@ struct Coarse {
   CoarseBlock cb;
 };
 
-// reduction scratch: partial sums + a completion counter per reduction slot
+// reduction scratch: partial sums of the blocks
 struct RedScratch {
-  double *partials = nullptr;   // RED_BLOCKS * 4
-  unsigned *counter = nullptr;  // one per slot
+  double *partials = nullptr;   // RED_BLOCKS * 2
   double *result = nullptr;     // result slots
 };
 
