@@ -119,7 +119,7 @@ __global__ __launch_bounds__(LU_T) void k_lu_wg(double *__restrict__ a, int n, i
       const int j = j0 + jj, par = jj & 1;
       double bv = (own && r >= j) ? fabs(rv[jj]) : -1.0;
       int bi = (own && r >= j) ? r : n;
-      wave_argmax(bv, bi);
+      wave_argmax<true>(bv, bi);
       if (lane == 0) {
         wv[par][wave] = bv;
         wi[par][wave] = bi;
@@ -131,21 +131,8 @@ __global__ __launch_bounds__(LU_T) void k_lu_wg(double *__restrict__ a, int n, i
 #pragma unroll
         for (int cc = 0; cc < LU_NB; ++cc) JB[par][cc] = rv[cc];
       __syncthreads();
-      {
-        // every wavefront's candidate loaded first, then taken in wavefront order
-        double cv[LU_T / 64];
-        int ci[LU_T / 64];
-#pragma unroll
-        for (int w2 = 0; w2 < LU_T / 64; ++w2) {
-          cv[w2] = wv[par][w2];
-          ci[w2] = wi[par][w2];
-        }
-        bv = cv[0];
-        bi = ci[0];
-#pragma unroll
-        for (int w2 = 1; w2 < LU_T / 64; ++w2) amax_take(bv, bi, cv[w2], ci[w2]);
-      }
-      const int p = bi;
+      block_argmax<LU_T / 64>(wv[par], wi[par], bv, bi);
+      const int p = bi < n ? bi : j;   // nothing but NaN in the column
       if (t == 0) {
         pivs[jj] = p;
         if (bv == 0.0 && info_s == 0) info_s = j + 1;

@@ -16,6 +16,7 @@
 #include "pmg_rows.hpp"
 #include "wave_argmax.hpp"
 #include "coarse_rows.hpp"
+#include <utility>
 
 namespace pmg {
 
@@ -76,6 +77,11 @@ __global__ void k_fill_d(double *x, double v, long n) {
   for (long i = blockIdx.x * long(blockDim.x) + threadIdx.x; i < n; i += long(gridDim.x) * blockDim.x) x[i] = v;
 }
 
+template <class F, int... J>
+__device__ inline __attribute__((always_inline)) void each_column(F &f, std::integer_sequence<int, J...>) {
+  (f(std::integral_constant<int, J>()), ...);
+}
+
 // Panel factorization of columns [j0, j1) (width <= NBR) with dgetf2 steps, the panel held
 // in registers (thread t owns rows j0 + t + PNT q, q < PR); two barriers per column (pivot
 // reduction, pivot row exchange), LDS double-buffered by column parity.  Then the panel's
@@ -100,8 +106,10 @@ __global__ __launch_bounds__(PT) void k_lu_panel(double *__restrict__ a, int n, 
 #pragma unroll
     for (int cc = 0; cc < NBR; ++cc) v[q][cc] = (r < n && cc < w) ? a[long(r) * n + j0 + cc] : 0.0;
   }
-#pragma unroll
-  for (int jj = 0; jj < NBR; ++jj) {
+  // a call per column, not a loop: PR = 7 passes the size up to which a loop is unrolled, and the
+  // panel would go from registers to scratch
+  auto step = [&](auto col) __attribute__((always_inline)) {
+    constexpr int jj = decltype(col)::value;
     if (jj < w) {
       const int j = j0 + jj, par = jj & 1;
       double bv = -1.0;
@@ -117,26 +125,14 @@ __global__ __launch_bounds__(PT) void k_lu_panel(double *__restrict__ a, int n, 
           }
         }
       }
-      wave_argmax(bv, bi);
+      wave_argmax<PR == 1>(bv, bi);
       if (lane == 0) {
         sv[par][wave] = bv;
         si[par][wave] = bi;
       }
       __syncthreads();
-      {
-        double cv[PT / 64];
-        int ci[PT / 64];
-#pragma unroll
-        for (int w2 = 0; w2 < PT / 64; ++w2) {
-          cv[w2] = sv[par][w2];
-          ci[w2] = si[par][w2];
-        }
-        bv = cv[0];
-        bi = ci[0];
-#pragma unroll
-        for (int w2 = 1; w2 < PT / 64; ++w2) amax_take(bv, bi, cv[w2], ci[w2]);
-      }
-      const int p = bi;
+      block_argmax<PT / 64>(sv[par], si[par], bv, bi);
+      const int p = bi < n ? bi : j;   // nothing but NaN in the column
       const bool nz = bv != 0.0;
       if (t == 0) {
         ipiv[j] = p;
@@ -178,7 +174,8 @@ __global__ __launch_bounds__(PT) void k_lu_panel(double *__restrict__ a, int n, 
         }
       }
     }
-  }
+  };
+  each_column(step, std::make_integer_sequence<int, NBR>());
 #pragma unroll
   for (int q = 0; q < PR; ++q) {
     const int r = j0 + t + PT * q;
