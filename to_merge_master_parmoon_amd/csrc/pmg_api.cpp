@@ -1100,7 +1100,7 @@ void vcycle_dev(pmg_ctx *c, const double *v, double *z) {
 void coarse_alloc(pmg_ctx *c, Coarse &C, int nr) {
   if (C.a && C.n != nr) {
     for (void *p : {(void *)C.a, (void *)C.f, (void *)C.ipiv, (void *)C.sigma, (void *)C.b, (void *)C.y,
-                    (void *)C.x, (void *)C.ubuf, (void *)C.swp, (void *)C.sync, (void *)C.flags})
+                    (void *)C.x, (void *)C.ubuf, (void *)C.swp, (void *)C.sync, (void *)C.words})
       dfree(c, p);
     C.a = nullptr;
   }
@@ -1115,11 +1115,10 @@ void coarse_alloc(pmg_ctx *c, Coarse &C, int nr) {
     C.x = dalloc<double>(c, C.n);
     C.ubuf = dalloc<double>(c, size_t(C.n) * 16);
     C.swp = dalloc<int>(c, 4 * 16 + 1);
-    const int nblk = (C.n + 63) / 64;
     C.sync = dalloc<unsigned>(c, 4);
-    C.flags = dalloc<unsigned>(c, 2 * size_t(nblk));
+    C.words = dalloc<unsigned long long>(c, 4 * size_t(C.n));
     PMG_HIP_CHECK(hipMemsetAsync(C.sync, 0, 4 * sizeof(unsigned), c->stream2));
-    PMG_HIP_CHECK(hipMemsetAsync(C.flags, 0, 2 * size_t(nblk) * sizeof(unsigned), c->stream2));
+    PMG_HIP_CHECK(hipMemsetAsync(C.words, 0, 4 * size_t(C.n) * sizeof(*C.words), c->stream2));
     if (!C.err) {
       C.err = dalloc<int>(c, 1);
       PMG_HIP_CHECK(hipMemsetAsync(C.err, 0, sizeof(int), c->stream2));

@@ -308,10 +308,11 @@ struct Coarse {
   double *b = nullptr;     // work vectors of the two sweeps
   double *y = nullptr;
   int *info = nullptr;
-  // triangular sweeps: generation + finish counter per sweep (4), per-row-block flags of the
-  // forward then the backward sweep (2 * ceil(n/64)), wait-limit error flag
-  unsigned *sync = nullptr, *flags = nullptr;
-  int *err = nullptr;
+  // triangular sweeps: generation + finish counter per sweep (4); per sweep the published values,
+  // two words of 32 bits and the generation each
+  unsigned *sync = nullptr;
+  unsigned long long *words = nullptr;
+  int *err = nullptr;   // set by a wait past its limit
   // the factorization runs on the second stream; the main stream waits for ev_done only
   // before the first coarse solve, and the pivot check happens at the next host sync
   hipEvent_t ev_start = nullptr, ev_done = nullptr;
