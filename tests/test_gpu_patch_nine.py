@@ -1,0 +1,45 @@
+"""One launch per color with nine velocity blocks (csrc/k_patch.hip): FP32 and BF16 sweeps against the
+oracle's FP64 sweep on boxes one coarse cell wide, colors of 1 to 8 cells, and faces with
+Dirichlet rows whose coupling blocks hold values that the sweep has to drop; then the same level
+with refinement steps, which take the two launches.  Bounds: FP32 rounding of the local
+inverses 2e-5, BF16's 2e-2, as with the shared block."""
+import numpy as np
+import pytest
+
+from conftest import params, rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("box,faces", [((1, 1, 1), 1), ((1, 1, 3), 21), ((3, 2, 2), 63), ((4, 4, 1), 21)])
+@pytest.mark.parametrize("precision,refine,bound", [(1, 0, 2e-5), (2, 0, 2e-2), (2, 1, 2e-2)])
+def test_nine_block_color_step(box, faces, precision, refine, bound):
+    import pmg_oracle
+    from to_merge_master_parmoon_amd import _abi, problem
+    from to_merge_master_parmoon_amd.multigrid import NSEMultiGrid
+    prob = problem.Problem(cx=box[0], cy=box[1], cz=box[2], n_levels=2, nu=0.1, conv_kind=_abi.CONV_FOURIER,
+                           rhs_kind=_abi.RHS_FOURIER, dirichlet_faces=faces, perturb=0.1)
+    rng = np.random.default_rng(6)
+    for lvl in range(2):
+        arr, d = prob.arrays(lvl), prob.descs[lvl]
+        ne, a = int(arr["a_rowptr"][d.n_active]), arr["a"]
+        a0 = a[0][:ne].copy()
+        for b, w in ((1, 0.05), (3, -0.05), (2, 0.03), (6, -0.03), (5, 0.02), (7, -0.02)):
+            a[b][:ne] = w * a0
+            a[b][ne:] = rng.standard_normal(len(a[b]) - ne)
+        a[4][:ne] = 1.1 * a0
+    prm = dict(internal_project_pressure=1 if faces == 63 else 0)
+    u = rng.standard_normal(prob.n_dof(1))
+    f = rng.standard_normal(prob.n_dof(1))
+    orc = pmg_oracle.Oracle(params(**prm), prob.descs, refactor=0)
+    x = u.copy()
+    assert orc.cell_vanka(1, x, f, 2) == 0
+    orc.close()
+    mg = NSEMultiGrid(params(precision=precision, bf16_refine_steps=refine, **prm))
+    for d in prob.descs:
+        mg.add_level(d)
+    mg.setup()
+    assert not mg.shared_block(1)
+    y = mg.cell_vanka(1, u.copy(), f, 2)
+    mg.close()
+    assert rel(y, x) <= bound

@@ -18,6 +18,12 @@
 // stored data), the two launches before and this one: 32^3 30.5 + 8.8 -> 20.4 us, 24^3 (full
 // inverses) 14.4 + 8.7 -> 13.0 us, 16^3 6.4 + 4.9 -> 6.2 us, 8^3 4.7 + 4.4 -> 4.4 us; the same
 // sums in the same order, so the same results bit for bit.
+//
+// With nine velocity blocks a patch streams 79 KB of rows and 29 KB of inverse (FP32): 512
+// patches of a 16^3 color take 12 us at the rate of a large copy.  A thread holds up to 99 row
+// values and 88 of the inverse; limited to 256 registers (24 bytes of scratch) two workgroups
+// share a CU.  Two launches before -> this one, FP32: 16^3 12.7 + 5.5 -> 12.3 us, 8^3
+// 5.6 + 4.7 -> 6.3 us, the same results bit for bit.
 #include "lu_sweeps.hpp"
 #include "pmg_internal.hpp"
 #include "pmg_rows.hpp"
@@ -111,7 +117,7 @@ struct VelRow<SH, 1> {
       for (int c = 0; c < 3; ++c) R.b[c][u] = v[c * R.n + clamp_entry(lane + 16 * u, R.n)];
     R.f = P.f[3L * P.N + d.w];
   }
-  __device__ __forceinline__ void residual(const float4 *hv, const float *, float *rs, int l64) const {
+  __device__ __forceinline__ float sum(const float4 *hv, int l64) const {
     const int lane = l64 & 15;
     const float4 y[2] = {hv[R.ib & 0xffffu], hv[R.ib >> 16]};
     float s = 0.0f;
@@ -121,8 +127,90 @@ struct VelRow<SH, 1> {
       const float z1 = ok ? y[u].x : 0.0f, z2 = ok ? y[u].y : 0.0f, z3 = ok ? y[u].z : 0.0f;
       s += fmaf(R.b[2][u], z3, fmaf(R.b[0][u], z1, R.b[1][u] * z2));   // as row_b_aos is compiled
     }
-    s = red16(s);
-    if (lane == 0 && R.row != PT_NOROW) rs[2 * NU_LOC + R.row] = R.f - s;
+    return red16(s);
+  }
+  __device__ __forceinline__ void residual(const float4 *hv, const float *, float *rs, int l64) const {
+    const float s = sum(hv, l64);
+    if ((l64 & 15) == 0 && R.row != PT_NOROW) rs[2 * NU_LOC + R.row] = R.f - s;
+  }
+};
+
+// velocity row of quad QD with nine velocity blocks, value b of entry j at 9 k0 + b n + j; the
+// local residual in the row order of the stored inverse (invperm)
+template <class SH, int QD>
+struct VelRow9 {
+  static constexpr int NA = SH::a(QD), NB = SH::bt(QD), OA = 64 * SH::off_a(QD), OB = 64 * SH::off_bt(QD);
+  int n, m, row, perm;
+  bool diag;   // Dirichlet row: the blocks A12 .. A32 are dropped
+  float a[9][NA], b[3][NB], f;
+  uint32_t ia[(NA + 1) / 2], ib;
+  __device__ __forceinline__ void load(const PatchStep &P, const int4 d, const uint32_t *__restrict__ pat,
+                                       const uint8_t *__restrict__ ip, int l64) {
+    const int lane = l64 & 15;
+    n = d.z & 255;
+    m = (d.z >> 8) & 255;
+    row = (d.z >> 16) & 255;
+    diag = d.w >= P.n_active;
+#pragma unroll
+    for (int p = 0; p < (NA + 1) / 2; ++p) ia[p] = pat[OA + 64 * p + l64];
+    ib = pat[OB + l64];
+    const float *v = P.av + 9L * d.x;
+#pragma unroll
+    for (int u = 0; u < NA; ++u)
+#pragma unroll
+      for (int c = 0; c < 9; ++c) a[c][u] = v[c * n + clamp_entry(lane + 16 * u, n)];
+    const float *w = P.btv + 3L * d.y;
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) b[c][u] = w[c * m + clamp_entry(lane + 16 * u, m)];
+    f = P.f[long(lane < 3 ? lane : 0) * P.N + d.w];
+    perm = ip[min(row + NU_LOC * (lane < 3 ? lane : 0), NLOC - 1)];
+  }
+  // sums in the order of row_a9_s (row_a_diag on Dirichlet rows) and row_bt_s
+  __device__ __forceinline__ void residual(const float4 *hv, const float *hp, float *rs, int l64) const {
+    const int lane = l64 & 15;
+    float4 y[NA];
+    float q[NB];
+#pragma unroll
+    for (int u = 0; u < NA; ++u) y[u] = hv[(ia[u / 2] >> (16 * (u % 2))) & 0xffffu];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) q[u] = hp[(ib >> (16 * u)) & 0xffffu];
+    float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < NA; ++u) {
+      const bool ok = lane + 16 * u < n;
+      const float z[3] = {ok ? y[u].x : 0.0f, ok ? y[u].y : 0.0f, ok ? y[u].z : 0.0f};
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const float all = s[r] + fmaf(a[3 * r + 2][u], z[2], fmaf(a[3 * r][u], z[0], a[3 * r + 1][u] * z[1]));
+        const float own = fmaf(a[4 * r][u], z[r], s[r]);
+        s[r] = diag ? own : all;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const float z = lane + 16 * u < m ? q[u] : 0.0f;
+#pragma unroll
+      for (int r = 0; r < 3; ++r) s[r] += b[r][u] * z;
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r) s[r] = red16(s[r]);
+    if (lane < 3 && row != PT_NOROW) rs[perm] = f - (lane == 0 ? s[0] : lane == 1 ? s[1] : s[2]);
+  }
+};
+template <class SH>
+struct VelRow9<SH, 1> {
+  VelRow<SH, 1> V;
+  int perm;
+  __device__ __forceinline__ void load(const PatchStep &P, const int4 d, const uint32_t *__restrict__ pat,
+                                       const uint8_t *__restrict__ ip, int l64) {
+    V.load(P, d, pat, l64);
+    perm = ip[min(V.R.row + 2 * NU_LOC, NLOC - 1)];
+  }
+  __device__ __forceinline__ void residual(const float4 *hv, const float *, float *rs, int l64) const {
+    const float s = V.sum(hv, l64);
+    if ((l64 & 15) == 0 && V.R.row != PT_NOROW) rs[perm] = V.R.f - s;
   }
 };
 
@@ -145,7 +233,7 @@ __device__ __forceinline__ void patch_barrier() {
 
 // The part of wavefront W: its two row quads, its share of the halo and of the stored data, then
 // of the local solve.
-template <typename F, bool FULL, bool GRID, int W>
+template <typename F, bool FULL, bool GRID, bool NINE, int W>
 __device__ __forceinline__ void patch_wave(const PatchStep &P, const F *__restrict__ stored, long pos, int l64,
                                            PatchLds<F, FULL> &S) {
   using SH = PatchShape<GRID>;
@@ -181,10 +269,16 @@ __device__ __forceinline__ void patch_wave(const PatchStep &P, const F *__restri
     h1 = ua[loc1];
     hq = P.u[3L * P.N + run + t % 4];
   }
-  VelRow<SH, 2 * W> A;
-  VelRow<SH, 2 * W + 1> B;
-  A.load(P, d0, pat, l64);
-  B.load(P, d1, pat, l64);
+  std::conditional_t<NINE, VelRow9<SH, 2 * W>, VelRow<SH, 2 * W>> A;
+  std::conditional_t<NINE, VelRow9<SH, 2 * W + 1>, VelRow<SH, 2 * W + 1>> B;
+  if constexpr (NINE) {
+    const uint8_t *__restrict__ ip = P.invperm + pos * PERM_STRIDE;
+    A.load(P, d0, pat, ip, l64);
+    B.load(P, d1, pat, ip, l64);
+  } else {
+    A.load(P, d0, pat, l64);
+    B.load(P, d1, pat, l64);
+  }
   if constexpr (W == 0) {
     own = pat[SH::own + min(t, NU_LOC - 1) / 2] >> (16 * (t & 1));
     pv = P.u[3L * P.N + (t < NU_LOC ? 0 : dof)];   // (lanes of velocity dofs: unused)
@@ -321,22 +415,22 @@ __device__ __forceinline__ int patch_slot(const Step &P) {
 }
 
 // FULL: stored 85 x 85 inverse (minv layout), else the block form (SCH_* layout).  GRID: shape
-// of the records' patterns.
-template <typename F, bool FULL, bool GRID>
-__global__ __launch_bounds__(256) void k_patch_step(PatchStep P, const F *__restrict__ stored) {
+// of the records' patterns.  NINE: nine velocity blocks, else the shared one.
+template <typename F, bool FULL, bool GRID, bool NINE>
+__global__ __launch_bounds__(256, NINE ? 2 : 1) void k_patch_step(PatchStep P, const F *__restrict__ stored) {
   __shared__ __align__(16) PatchLds<F, FULL> S;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l64 = threadIdx.x & 63;
   const int slot = patch_slot(P);
   if (slot < 0) return;
   const long pos = long(P.pos0) + slot;
   if (wave == 0)
-    patch_wave<F, FULL, GRID, 0>(P, stored, pos, l64, S);
+    patch_wave<F, FULL, GRID, NINE, 0>(P, stored, pos, l64, S);
   else if (wave == 1)
-    patch_wave<F, FULL, GRID, 1>(P, stored, pos, l64, S);
+    patch_wave<F, FULL, GRID, NINE, 1>(P, stored, pos, l64, S);
   else if (wave == 2)
-    patch_wave<F, FULL, GRID, 2>(P, stored, pos, l64, S);
+    patch_wave<F, FULL, GRID, NINE, 2>(P, stored, pos, l64, S);
   else
-    patch_wave<F, FULL, GRID, 3>(P, stored, pos, l64, S);
+    patch_wave<F, FULL, GRID, NINE, 3>(P, stored, pos, l64, S);
 }
 
 // ------------------------------------------------------------------ FP64
@@ -580,11 +674,17 @@ void launch_patch_step(const PatchStep &P, const float *stored32, const uint16_t
   auto go = [&](auto f_c, const auto *stored) {
     constexpr bool FULL = decltype(f_c)::value;
     using F = std::remove_const_t<std::remove_pointer_t<decltype(stored)>>;
+    if constexpr (FULL)
+      if (P.av) {
+        k_patch_step<F, true, true, true><<<grid, 256, 0, s>>>(P, stored);
+        return;
+      }
     if (P.grid)
-      k_patch_step<F, FULL, true><<<grid, 256, 0, s>>>(P, stored);
+      k_patch_step<F, FULL, true, false><<<grid, 256, 0, s>>>(P, stored);
     else
-      k_patch_step<F, FULL, false><<<grid, 256, 0, s>>>(P, stored);
+      k_patch_step<F, FULL, false, false><<<grid, 256, 0, s>>>(P, stored);
   };
+  if (P.av && !(full && P.grid)) throw DeviceError("launch_patch_step: nine blocks without full inverses on a grid");
   if (stored16 && full)
     go(std::true_type{}, stored16);
   else if (stored16)

@@ -608,12 +608,16 @@ void nodal_sweep(pmg_ctx *c, DevLevel &D, double *u, const double *f, double *au
   if (last) set_dirichlet(c, D, u, f);
 }
 
+// the FP32 sweep with nine velocity blocks in one launch per color (k_patch.hip)
+bool fused_nine(const pmg_ctx *c, const DevLevel &D) {
+  return !D.a_shared && D.patch_rec && D.patch_grid && !D.schur && c->prm.bf16_refine_steps == 0;
+}
 // the interleaved velocity copy a level's FP32 sweeps gather from (stored inverses and the
-// shared velocity block), or null
+// shared velocity block or the fused launch), or null
 template <typename T>
-float *sweep_copy(const DevLevel &D) {
+float *sweep_copy(const pmg_ctx *c, const DevLevel &D) {
   if constexpr (sizeof(T) == 4) {
-    if (D.ua32 && D.a_shared && (D.minv16 || D.minv32)) return D.ua32;
+    if (D.ua32 && (D.a_shared || fused_nine(c, D)) && (D.minv16 || D.minv32)) return D.ua32;
   }
   return nullptr;
 }
@@ -649,7 +653,7 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   const int fb = sizeof(T) == 8 ? 8 : (c->prm.precision == PMG_PREC_FP32_BF16 ? 2 : 4);
   // FP32 with inverses and the shared block: the residual gathers the velocity from the
   // interleaved copy ua, built here and kept current by the local updates
-  float *ua = sweep_copy<T>(D);
+  float *ua = sweep_copy<T>(c, D);
   if (!started) {
     if (ua && !(first == false && !relax))
       launch_sweep_start(reinterpret_cast<float *>(u), reinterpret_cast<const float *>(f), D.n_udof, D.hanging_bound,
@@ -662,8 +666,8 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   const int nref = sizeof(T) == 4 ? c->prm.bf16_refine_steps : 0;
   // one launch per color: residual, local solve and update of a patch by one workgroup, at every
   // size faster than the two launches (k_patch.hip); these stay for refinement steps, nine
-  // blocks, stored LU factors and levels whose patches fit no record (rows of more than 128
-  // entries, shared pressure dofs, colors that share dofs)
+  // blocks in FP64 or off a hexahedral grid, stored FP32 LU factors and levels whose patches fit
+  // no record (rows of more than 128 entries, shared pressure dofs, colors that share dofs)
   const bool fused = sizeof(T) == 8 ? rloc == reinterpret_cast<T *>(D.rloc) && D.patch_rec && D.a_shared
                                     : ua && D.patch_rec && nref == 0;
   const bool full = !D.schur;
@@ -689,11 +693,12 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
       if (fused) {
         const double sb = full ? double(MINV_STRIDE) : double(SCH_STRIDE);
         // the rows of the residual, the stored data, the record, the new values
-        const double by = D.res_bytes[1][1][col] * part - nc * (31.0 * 20 + 2 * 85 * 4.0) +
+        const double by = D.res_bytes[D.a_shared][1][col] * part - nc * (31.0 * 20 + 2 * 85 * 4.0) +
                           nc * (sb * fb + 4.0 * D.patch_stride + 27 * 16.0 + 32);
         Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
         PatchStep P{D.patch_rec, D.patch_pat, slots, op.a1, op.btv, op.bv, f, u, ua, damp, D.patch_stride, D.n_udof,
-                    nc, p0, nc >= XCD_GROUP_MIN && D.tune_res_xcd[1], full, D.patch_grid};
+                    nc, p0, nc >= XCD_GROUP_MIN && D.tune_res_xcd[1], full, D.patch_grid, D.a_shared ? nullptr : op.av,
+                    D.invperm, op.n_active};
         launch_patch_step(P, D.minv32, D.minv16, full, c->stream);
         continue;
       }
@@ -955,7 +960,7 @@ void cycle(pmg_ctx *c, int i, bool zero) {
   bool started = false;
   if (zero) {
     if (i > 0 && c->prm.sc_pre_smooth_saddle > 0 && !D.nodal && D.coarse_insts.empty()) {
-      launch_start_zero<T>(u, f, D.n_udof, D.n_pdof, D.hanging_bound, D.n_dirichlet, sweep_copy<T>(D), c->stream);
+      launch_start_zero<T>(u, f, D.n_udof, D.n_pdof, D.hanging_bound, D.n_dirichlet, sweep_copy<T>(c, D), c->stream);
       started = true;
     } else if (i > 0 || c->batch) {
       launch_fill<T>(u, T(0), D.n_dof, c->stream);
@@ -1002,7 +1007,7 @@ void cycle(pmg_ctx *c, int i, bool zero) {
       Timed tm(c, &c->tm.transfer, D.transfer_bytes, 0.0);
       const bool sub = D.act_lists;
       launch_prolong_update<T>(D.pu, D.pp, Vec<T>::sol(C), C.n_udof, u, D.n_udof, damp, f, D.hanging_bound,
-                               D.n_dirichlet, sweep_copy<T>(D), c->stream, sub ? D.act_u : nullptr, D.n_act_u,
+                               D.n_dirichlet, sweep_copy<T>(c, D), c->stream, sub ? D.act_u : nullptr, D.n_act_u,
                                sub ? D.act_p : nullptr, D.n_act_p);
     }
     for (int j = 0; j < post; ++j)

@@ -399,6 +399,9 @@ struct PatchStep {
   int grouped;                // 1: consecutive patches of the color per XCD
   int mirror;                 // 1: u takes the new velocity too
   int grid;                   // PatchShape<true>, else <false>
+  const float *av;            // nine velocity blocks (grid and full inverses only), null: the shared one
+  const uint8_t *invperm;     // (nine blocks) row order of the stored inverses
+  int n_active;
 };
 // the same of the FP64 sweep with the shared block and stored LU factors; alt: the copies of the
 // velocity after u itself, three component vectors of N each
