@@ -38,21 +38,30 @@ __device__ inline void q2_at(int q, int i, double &v, double &dx, double &dy, do
   dz = vx[a] * vy[b] * az[c];
 }
 
-// zero the nine A blocks of the active rows (entries [0, a_rowptr[n_active]))
-__global__ void k_zero_active(double *__restrict__ a, long nnz, long n_act_entries) {
-  for (long k = blockIdx.x * long(blockDim.x) + threadIdx.x; k < 9 * n_act_entries;
-       k += long(gridDim.x) * blockDim.x) {
-    const long b = k / n_act_entries, e = k - b * n_act_entries;
-    a[b * nnz + e] = 0.0;
+// block 0 of the active rows (entries [0, a_rowptr[n_active])) to zero before the colors add to it
+__global__ void k_zero_active(double *__restrict__ a, long n_act_entries) {
+  for (long k = blockIdx.x * long(blockDim.x) + threadIdx.x; k < n_act_entries; k += long(gridDim.x) * blockDim.x)
+    a[k] = 0.0;
+}
+// the other eight blocks after them: A22 = A33 = A11, the rest zero.  The colors add to one block
+// only (three would be 107 MB read and written per color of 3072 cells), and this pass writes what
+// the zeroing of nine blocks wrote before: 16 us as before at 24576 cells.
+__global__ void k_spread_active(double *__restrict__ a, long nnz, long n_act_entries) {
+  for (long k = blockIdx.x * long(blockDim.x) + threadIdx.x; k < n_act_entries; k += long(gridDim.x) * blockDim.x) {
+    const double v = a[k];
+#pragma unroll
+    for (int b = 1; b < 9; ++b) a[b * nnz + k] = b % 4 == 0 ? v : 0.0;
   }
 }
 
 // Geometry and basis data of one cell in LDS: weights w_q |det J| (W), values Vq[q][i] and
 // physical gradients G*[q][i] of the 27 Q2 basis functions at the 27 Gauss points, and the
-// convection at the points (Bc).  Called by all 256 threads; ends with a barrier.
+// convection at the points (Bc) and times the gradients (Bg).  Called by all CELL_T threads;
+// ends with a barrier.
+constexpr int CELL_T = 128;
 struct CellData {
   double X[8][3], Bc[27][3], Ji[27][9], W[27];
-  double Vq[27][27], Gx[27][27], Gy[27][27], Gz[27][27];
+  double Vq[27][27], Gx[27][27], Gy[27][27], Gz[27][27], Bg[27][27];
 };
 
 __device__ void cell_setup(CellData &D, int cell, const double *__restrict__ geom, const double *__restrict__ bq) {
@@ -94,86 +103,134 @@ __device__ void cell_setup(CellData &D, int cell, const double *__restrict__ geo
   }
   __syncthreads();
   // physical gradients: J^{-T} times the reference gradient
-  for (int idx = t; idx < 27 * 27; idx += 256) {
+  for (int idx = t; idx < 27 * 27; idx += CELL_T) {
     const int q = idx / 27, i = idx - 27 * q;
     double v, dx, dy, dz;
     q2_at(q, i, v, dx, dy, dz);
     const double *I = D.Ji[q];
+    const double gx = I[0] * dx + I[3] * dy + I[6] * dz;
+    const double gy = I[1] * dx + I[4] * dy + I[7] * dz;
+    const double gz = I[2] * dx + I[5] * dy + I[8] * dz;
     D.Vq[q][i] = v;
-    D.Gx[q][i] = I[0] * dx + I[3] * dy + I[6] * dz;
-    D.Gy[q][i] = I[1] * dx + I[4] * dy + I[7] * dz;
-    D.Gz[q][i] = I[2] * dx + I[5] * dy + I[8] * dz;
+    D.Gx[q][i] = gx;
+    D.Gy[q][i] = gy;
+    D.Gz[q][i] = gz;
+    D.Bg[q][i] = D.Bc[q][0] * gx + D.Bc[q][1] * gy + D.Bc[q][2] * gz;
   }
   __syncthreads();
 }
 
-// element entry (test i, ansatz j) of NSType4Galerkin3D with the mass term sigma
-__device__ inline double element_entry(const CellData &D, int i, int j, double nu, double sigma) {
-  double s = 0.0;
+// Element entries (test i, ansatz j) of NSType4Galerkin3D with the mass term sigma: thread t < 81 takes
+// the nine with i = t / 9 + 9 r, j = t % 9 + 9 c.
+// Bounds: one entry per thread at a time read eleven values from LDS per point and entry and,
+// unrolled over the points, took the whole register file, so one cell was in work per CU and
+// waited at each of its steps; nine per thread read three, and five cells share a CU.  3072 cells:
+// k_assemble_oseen 248 -> 76 us, k_theta_rhs 172 -> 65 us, the same values bit for bit.
+constexpr int TILES = 81;
+__device__ __forceinline__ void element_entries(const CellData &D, int t, double nu, double sigma, double (&s)[3][3]) {
+  const int i0 = t / 9, j0 = t - 9 * i0;
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) s[r][c] = 0.0;
+#pragma unroll 1
   for (int q = 0; q < 27; ++q) {
-    double val = nu * (D.Gx[q][i] * D.Gx[q][j] + D.Gy[q][i] * D.Gy[q][j] + D.Gz[q][i] * D.Gz[q][j]);
-    val += (D.Bc[q][0] * D.Gx[q][j] + D.Bc[q][1] * D.Gy[q][j] + D.Bc[q][2] * D.Gz[q][j]) * D.Vq[q][i];
-    if (sigma != 0.0) val += sigma * D.Vq[q][j] * D.Vq[q][i];
-    s += D.W[q] * val;
+    const double w = D.W[q];
+    double xi[3], yi[3], zi[3], vi[3], xj[3], yj[3], zj[3], vj[3], bj[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      xi[r] = D.Gx[q][i0 + 9 * r];
+      yi[r] = D.Gy[q][i0 + 9 * r];
+      zi[r] = D.Gz[q][i0 + 9 * r];
+      vi[r] = D.Vq[q][i0 + 9 * r];
+      xj[r] = D.Gx[q][j0 + 9 * r];
+      yj[r] = D.Gy[q][j0 + 9 * r];
+      zj[r] = D.Gz[q][j0 + 9 * r];
+      vj[r] = D.Vq[q][j0 + 9 * r];
+      bj[r] = D.Bg[q][j0 + 9 * r];
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        double val = fma(nu, fma(zi[r], zj[c], fma(xi[r], xj[c], yi[r] * yj[c])), bj[c] * vi[r]);
+        if (sigma != 0.0) val = fma(sigma * vj[c], vi[r], val);
+        s[r][c] = fma(w, val, s[r][c]);
+      }
   }
-  return s;
 }
 
-__global__ __launch_bounds__(256) void k_assemble_oseen(const int *__restrict__ cells, int ncells,
-                                                        const double *__restrict__ geom,
-                                                        const double *__restrict__ bq,
-                                                        const int *__restrict__ u_global,
-                                                        const int *__restrict__ pmap,
-                                                        const int *__restrict__ a_rowptr, int n_active, long nnz,
-                                                        double *__restrict__ a, double nu, double sigma) {
+__global__ __launch_bounds__(CELL_T) void k_assemble_oseen(const int *__restrict__ cells, int ncells,
+                                                           const double *__restrict__ geom,
+                                                           const double *__restrict__ bq,
+                                                           const int *__restrict__ u_global,
+                                                           const int *__restrict__ pmap,
+                                                           const int *__restrict__ a_rowptr, int n_active,
+                                                           double *__restrict__ a, double nu, double sigma) {
   __shared__ CellData D;
   if (int(blockIdx.x) >= ncells) return;
-  const int cell = cells[blockIdx.x];
-  cell_setup(D, cell, geom, bq);
+  const int cell = cells[blockIdx.x], t = threadIdx.x;
   const int *ug = u_global + long(cell) * NU_LOC;
   const int *mp = pmap + long(cell) * PM_STRIDE;
-  for (int idx = threadIdx.x; idx < 27 * 27; idx += 256) {
-    const int i = idx / 27, j = idx - 27 * i;
-    const int row = ug[i];
-    if (row >= n_active) continue;   // Dirichlet rows keep their identity
-    const double s = element_entry(D, i, j, nu, sigma);
-    // entry (row, col j) in the CSR: the gather map holds its row-blocked offset
-    // 9 k0 + (k - k0) of block 0
-    const int off = mp[PM_A + i * NU_LOC + j];
-    if (off < 0) continue;
-    const long k = long(off) - 8L * a_rowptr[row];
-    a[k] += s;
-    a[4 * nnz + k] += s;
-    a[8 * nnz + k] += s;
+  // entry (row, col j) in the CSR: the gather map holds its row-blocked offset 9 k0 + (k - k0) of
+  // block 0; Dirichlet rows keep their identity
+  long k[3][3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int i = min(t, TILES - 1) / 9 + 9 * r, row = ug[i];
+    const long k0 = row < n_active ? 8L * a_rowptr[row] : 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int off = mp[PM_A + i * NU_LOC + min(t, TILES - 1) % 9 + 9 * c];
+      k[r][c] = t < TILES && row < n_active && off >= 0 ? off - k0 : -1;
+    }
   }
+  cell_setup(D, cell, geom, bq);
+  if (t >= TILES) return;
+  double s[3][3], old[3][3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) old[r][c] = k[r][c] >= 0 ? a[k[r][c]] : 0.0;
+  element_entries(D, t, nu, sigma, s);
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (k[r][c] >= 0) a[k[r][c]] = old[r][c] + s[r][c];
 }
 
 // rhs_c(row i) -= sum_j E_ij(nu, sigma') u_c(j) for the active rows of one color's cells:
 // with sigma' = -sigma, sigma M u - A u of the theta scheme's right-hand side
-__global__ __launch_bounds__(256) void k_theta_rhs(const int *__restrict__ cells, int ncells,
-                                                   const double *__restrict__ geom, const double *__restrict__ bq,
-                                                   const int *__restrict__ u_global, int n_udof, int n_active,
-                                                   const double *__restrict__ u, double *__restrict__ rhs, double nu,
-                                                   double sigma_neg) {
+__global__ __launch_bounds__(CELL_T) void k_theta_rhs(const int *__restrict__ cells, int ncells,
+                                                      const double *__restrict__ geom, const double *__restrict__ bq,
+                                                      const int *__restrict__ u_global, int n_udof, int n_active,
+                                                      const double *__restrict__ u, double *__restrict__ rhs,
+                                                      double nu, double sigma_neg) {
   __shared__ CellData D;
-  __shared__ double E[27][28];
+  __shared__ double ul[81];
   if (int(blockIdx.x) >= ncells) return;
-  const int cell = cells[blockIdx.x];
-  cell_setup(D, cell, geom, bq);
-  for (int idx = threadIdx.x; idx < 27 * 27; idx += 256) {
-    const int i = idx / 27, j = idx - 27 * i;
-    E[i][j] = element_entry(D, i, j, nu, sigma_neg);
-  }
-  __syncthreads();
+  const int cell = cells[blockIdx.x], t = threadIdx.x;
   const int *ug = u_global + long(cell) * NU_LOC;
-  const int t = threadIdx.x;
+  if (t < 81) ul[t] = u[long(t / 27) * n_udof + ug[t % 27]];
+  cell_setup(D, cell, geom, bq);
+  double s[3][3];
+  if (t < TILES) element_entries(D, t, nu, sigma_neg, s);
+  __syncthreads();
+  double(*const E)[27] = D.Gx;   // no longer needed
+  if (t < TILES)
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) E[t / 9 + 9 * r][t % 9 + 9 * c] = s[r][c];
+  __syncthreads();
   if (t < 81) {
     const int i = t / 3, c = t - 3 * i;
     const int row = ug[i];
     if (row < n_active) {
-      double s = 0.0;
-      for (int j = 0; j < 27; ++j) s += E[i][j] * u[long(c) * n_udof + ug[j]];
-      rhs[long(c) * n_udof + row] -= s;
+      double v = 0.0;
+      for (int j = 0; j < 27; ++j) v += E[i][j] * ul[27 * c + j];
+      rhs[long(c) * n_udof + row] -= v;
     }
   }
 }
@@ -222,15 +279,17 @@ void launch_assemble_oseen(const DevLevel &L, const double *geom, const double *
   PMG_HIP_CHECK(hipMemcpyAsync(rp.data(), L.a_rowptr + L.n_active, sizeof(int), hipMemcpyDeviceToHost, s));
   PMG_HIP_CHECK(hipStreamSynchronize(s));
   const long n_act = rp[0];
-  k_zero_active<<<2048, 256, 0, s>>>(L.a, L.a_nnz, n_act);
+  k_zero_active<<<2048, 256, 0, s>>>(L.a, n_act);
   PMG_HIP_CHECK(hipGetLastError());
   for (int col = 0; col + 1 < int(L.ptr_colors.size()); ++col) {
     const int p0 = L.ptr_colors[col], nc = L.ptr_colors[col + 1] - p0;
     if (nc <= 0) continue;
-    k_assemble_oseen<<<nc, 256, 0, s>>>(L.cell_reorder + p0, nc, geom, bq, L.u_global, L.pmap, L.a_rowptr, L.n_active,
-                                        L.a_nnz, L.a, nu, sigma);
+    k_assemble_oseen<<<nc, CELL_T, 0, s>>>(L.cell_reorder + p0, nc, geom, bq, L.u_global, L.pmap, L.a_rowptr,
+                                           L.n_active, L.a, nu, sigma);
     PMG_HIP_CHECK(hipGetLastError());
   }
+  k_spread_active<<<2048, 256, 0, s>>>(L.a, L.a_nnz, n_act);
+  PMG_HIP_CHECK(hipGetLastError());
 }
 
 void launch_theta_rhs(const DevLevel &L, const double *geom, const double *bq, double nu, double sigma,
@@ -241,7 +300,7 @@ void launch_theta_rhs(const DevLevel &L, const double *geom, const double *bq, d
   for (int col = 0; col + 1 < int(L.ptr_colors.size()); ++col) {
     const int p0 = L.ptr_colors[col], nc = L.ptr_colors[col + 1] - p0;
     if (nc <= 0) continue;
-    k_theta_rhs<<<nc, 256, 0, s>>>(L.cell_reorder + p0, nc, geom, bq, L.u_global, L.n_udof, L.n_active, u, rhs, nu,
+    k_theta_rhs<<<nc, CELL_T, 0, s>>>(L.cell_reorder + p0, nc, geom, bq, L.u_global, L.n_udof, L.n_active, u, rhs, nu,
                                    -sigma);
     PMG_HIP_CHECK(hipGetLastError());
   }
