@@ -458,10 +458,11 @@ void drop_graph(pmg_ctx *c);
 void ensure_xa(pmg_ctx *c);
 
 void refresh_values(pmg_ctx *c, DevLevel &D) {
-  launch_row_blocked<double>(D, D.av64, D.bv64, D.btv64, c->stream);
-  if (D.av32) launch_row_blocked<float>(D, D.av32, D.bv32, D.btv32, c->stream);
   const bool was = D.a_shared;
   D.a_shared = c->prm.shared_block && shared_velocity_block(D, c->red.partials, c->stream);
+  // (after the check: with the shared block only one of the nine is copied)
+  launch_row_blocked<double>(D, D.av64, D.bv64, D.btv64, c->stream);
+  if (D.av32) launch_row_blocked<float>(D, D.av32, D.bv32, D.btv32, c->stream);
   // the captured V-cycle holds the kernels and operator views of the previous form
   if (D.a_shared != was) drop_graph(c);
   if (D.a_shared && D.av32) {
