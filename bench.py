@@ -354,9 +354,9 @@ def run_channel(args, log):
 def measured_traffic(kernel: str, precision: str, n: int):
     """HBM bytes per launch of `kernel` on the finest level from the committed rocprofv3
     FETCH_SIZE/WRITE_SIZE summary (calibrated against a copy kernel)."""
-    if precision not in ("fp32", "bf16") or n != 32:   # the mixed paths share k_vanka_res<float>
+    if precision not in ("fp32", "bf16") or n != 32:   # only those are profiled
         return None, None
-    path = ROOT / "profiles" / f"k_vanka_res_oseen32_{precision}_hbm_traffic.md"
+    path = ROOT / "profiles" / f"{kernel}_oseen32_{precision}_hbm_traffic.md"
     if not path.exists():
         return None, None
     for line in path.read_text().splitlines():
@@ -389,7 +389,7 @@ def general_type4_res_bytes(prob, vs: int = 4) -> float:
 
 
 def roofline_from(tm: dict, precision: str, n: int, prob):
-    """Roofline of the finest level's local-residual kernel from the profiling pass."""
+    """Roofline of the finest level's color step (residual, local solve, update) from the profiling pass."""
     kern = {k: v for k, v in tm.items() if isinstance(v, dict) and v["calls"] > 0}
     v = tm["vanka_res_finest"]
     avg_ms = v["ms"] / v["calls"]
@@ -400,13 +400,13 @@ def roofline_from(tm: dict, precision: str, n: int, prob):
                          avg_us=round(1e3 * x["ms"] / x["calls"], 2),
                          gbs=round(x["bytes"] / (x["ms"] * 1e-3) / 1e9, 1) if x["ms"] > 0 else None)
                  for k, x in kern.items()}
-    traffic, src = measured_traffic("k_vanka_res", precision, n)
-    roof = {"bound": "hbm", "kernel": "k_vanka_res (finest level, one color per launch)",
+    traffic, src = measured_traffic("k_patch_step", precision, n)
+    roof = {"bound": "hbm", "kernel": "k_patch_step (finest level, one color per launch)",
             "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None if traffic is None else round(traffic),
             "bytes_per_launch": round(bytes_per_launch), "avg_launch_us": round(avg_ms * 1e3, 2),
-            # the same launch's bytes in the general type-4 format (nine A values per entry,
-            # no credit for equal or vanishing blocks): what the nine-block kernel streams
+            # the residual's bytes alone in the general type-4 format (nine A values per entry,
+            # no credit for equal or vanishing blocks)
             "bytes_per_launch_general_type4": round(gen)}
     if src:
         roof["traffic_source"] = src
@@ -606,10 +606,10 @@ def main():
                 nine_res = r["timers"]["vanka_res_finest"]
         cfg["nine_blocks"] = {f"{k}_solve_s": round(v / 1e3, 5) for k, v in nine.items()}
         if nine_res and nine_res["calls"]:
-            # the nine-block residual kernel streams the general type-4 bytes itself
+            # the nine-block color step streams the general type-4 bytes itself
             us = 1e3 * nine_res["ms"] / nine_res["calls"]
             b = nine_res["bytes"] / nine_res["calls"]
-            cfg["nine_blocks"]["k_vanka_res_finest"] = {"avg_launch_us": round(us, 2), "bytes_per_launch": round(b),
+            cfg["nine_blocks"]["k_patch_step_finest"] = {"avg_launch_us": round(us, 2), "bytes_per_launch": round(b),
                                                         "achieved_gbs": round(b / us / 1e3, 1),
                                                         "frac": round(b / us / 1e3 / HBM_PEAK_GBS, 4)}
         if prec and ref is not None:

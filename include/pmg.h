@@ -388,14 +388,15 @@ typedef struct {
 typedef struct {
   pmg_kstat defect;        /* k_type4 in the V-cycle and the level defect                */
   pmg_kstat matvec;        /* k_type4 as FGMRES operator / Defect_NSE4                    */
-  pmg_kstat vanka_res;     /* per-color local residuals                                   */
-  pmg_kstat vanka_solve;   /* per-color stored-factor local solves + update               */
+  pmg_kstat vanka_res;     /* per-color launches: residual, solve and update, or (two-launch
+                              form) the local residuals                                   */
+  pmg_kstat vanka_solve;   /* (two-launch form) per-color local solves + update           */
   pmg_kstat transfer;      /* restriction + prolongation SpMVs                            */
   pmg_kstat coarse_solve;  /* coarse triangular sweeps                                    */
   pmg_kstat patch_lu;      /* batched patch LU (set-up)                                   */
   pmg_kstat coarse_lu;     /* coarse dense LU (set-up)                                    */
   double sweep_ms; long long sweep_calls;   /* whole colored sweeps                       */
-  pmg_kstat vanka_res_finest;  /* the per-color local residuals of the finest level alone */
+  pmg_kstat vanka_res_finest;  /* vanka_res of the finest level alone                     */
 } pmg_timers;
 /* Launch-shape autotuner (no reference counterpart; the reference's kernels have fixed
    shapes): after pmg_setup, times the candidate launch shapes of every smoothed level's

@@ -694,7 +694,7 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
       if (fused) {
         const double sb = full ? double(MINV_STRIDE) : double(SCH_STRIDE);
         // the rows of the residual, the stored data, the record, the new values
-        const double by = D.res_bytes[D.a_shared][1][col] * part - nc * (31.0 * 20 + 2 * 85 * 4.0) +
+        const double by = (D.res_bytes[D.a_shared][1][col] - D.res_index_bytes[col]) * part - nc * (31.0 * 20 + 2 * 85 * 4.0) +
                           nc * (sb * fb + 4.0 * D.patch_stride + 27 * 16.0 + 32);
         Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
         PatchStep P{D.patch_rec, D.patch_pat, slots, op.a1, op.btv, op.bv, f, u, ua, damp, D.patch_stride, D.n_udof,
@@ -704,7 +704,7 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
         continue;
       }
     } else if (fused) {
-      const double by = D.res_bytes[1][0][col] * part - nc * (31.0 * 20 + 85 * 8.0) +
+      const double by = (D.res_bytes[1][0][col] - D.res_index_bytes[col]) * part - nc * (31.0 * 20 + 85 * 8.0) +
                         nc * (NLOC * NLOC * 8.0 + 4.0 * D.patch_stride + 85 * 8.0);
       Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
       PatchStep64 P{D.patch_rec, D.patch_pat, slots, D.invperm, op.a1, op.btv, op.bv, f, D.lu, u, D.patch_alt, damp,
@@ -2205,6 +2205,20 @@ static int add_level(pmg_ctx *c, const pmg_level_desc *d, int *level_out, bool m
               for (int j = 0; j < NP_LOC; ++j) b += rb.pre(d, pg[size_t(cell) * NP_LOC + j], vs) - 8 + vs + vs + uo + 1;
             }
             D.res_bytes[sh][pi][k] = b;
+          }
+        }
+      // the column indices in them, which the one-launch form replaces by shared patterns
+      D.res_index_bytes.assign(nc, 0.0);
+      for (int k = 0; k < nc; ++k)
+        for (int q = ptr[k]; q < ptr[k + 1]; ++q) {
+          for (int j = 0; j < NU_LOC; ++j) {
+            const int g = ug[size_t(reo[q]) * NU_LOC + j];
+            D.res_index_bytes[k] += 4.0 * (d->a_rowptr[g + 1] - d->a_rowptr[g]);
+            if (g < d->n_active) D.res_index_bytes[k] += 4.0 * (d->bt_rowptr[g + 1] - d->bt_rowptr[g]);
+          }
+          for (int j = 0; j < NP_LOC; ++j) {
+            const int g = pg[size_t(reo[q]) * NP_LOC + j];
+            D.res_index_bytes[k] += 4.0 * (d->b_rowptr[g + 1] - d->b_rowptr[g]);
           }
         }
     }

@@ -208,7 +208,7 @@ struct DevLevel {
   // algorithmic bytes (FP64 operator) of the per-color residual launches and of one defect
   // [0]: FP64 values and vectors, [1]: FP32
   // [s][p]: s = 1 with the shared velocity block, p = 0 FP64, 1 FP32
-  std::vector<double> res_bytes[2][2];
+  std::vector<double> res_bytes[2][2], res_index_bytes;
   double defect_bytes[2][2] = {{0, 0}, {0, 0}}, matvec_bytes[2] = {0, 0};
   double transfer_bytes = 0;
   // merged (batched) levels: the problems solved directly on this level, and the
