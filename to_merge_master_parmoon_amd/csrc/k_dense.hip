@@ -451,28 +451,41 @@ __global__ __launch_bounds__(256) void k_trsv_chain(const double *__restrict__ f
   __syncthreads();
   if (qd == 0) {
     double v = r < kb ? b0 - ((part[0][r] + part[1][r]) + (part[2][r] + part[3][r])) : 0.0;
-    if (!UPPER) {
+    // Every lane forms the corrected quotient of its row at each step and lane k's is used:
+    // q = x rc, e = fma(-q, u, x), q' = fma(e, rc, q), which with rc = RN(1/u) is the correctly
+    // rounded x / u (Markstein); a lower sweep divides by nothing.
+    auto quotient = [&](double y) {
+      if (!UPPER) return y;
+      const double q = y * rc;
+      return fma(fma(-q, dg, y), rc, q);
+    };
+    // A row does not change after its own step (its entries are zero from there on), so after the
+    // last one its quotient is its solution.
+    double z = v;
 #pragma unroll
-      for (int k = 0; k < TB; ++k) v = fma(-bcast(v, k), row_v[k], v);
-    } else {
-      // Every lane forms the corrected quotient of its row at each step and lane k's is used:
-      // q = x rc, e = fma(-q, u, x), q' = fma(e, rc, q), which with rc = RN(1/u) is the correctly
-      // rounded x / u (Markstein).  A row does not change after its own step, so after the last
-      // one the quotient is its solution.
-      auto quotient = [&](double z) {
-        const double q = z * rc;
-        return fma(fma(-q, dg, z), rc, q);
-      };
-#pragma unroll
-      for (int k = TB - 1; k >= 0; --k) v = fma(-bcast(quotient(v), k), row_v[k], v);
-      v = quotient(v);
+    for (int i = 0; i < TB; ++i) {
+      const int k = UPPER ? TB - 1 - i : i;
+      z = fma(-bcast(quotient(z), k), row_v[k], z);
+    }
+    z = quotient(z);
+    // unless one of the unknowns is not finite, which zero times it would carry to the finished rows
+    // (and which its own row shows at the end): again with selects
+    if (__any(r < kb && !(fabs(z) < INFINITY))) {
+      z = v;
+#pragma unroll 1
+      for (int i = 0; i < kb; ++i) {
+        const int k = UPPER ? kb - 1 - i : i;
+        const double q = quotient(z), xk = bcast(q, k);
+        if (r == k) z = q;
+        if (r < kb && (UPPER ? r < k : r > k)) z = fma(-xk, f[long(R0 + k) * n + row], z);
+      }
     }
     if (r < kb) {
       const unsigned long long tag = (unsigned long long)gen << 32;
       unsigned long long *const wp = words + 2L * (R0 + r);
-      __hip_atomic_store(wp, tag | unsigned(__double2loint(v)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(wp + 1, tag | unsigned(__double2hiint(v)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      x[R0 + r] = v;
+      __hip_atomic_store(wp, tag | unsigned(__double2loint(z)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(wp + 1, tag | unsigned(__double2hiint(z)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      x[R0 + r] = z;
     }
   }
   if (t == 0) {

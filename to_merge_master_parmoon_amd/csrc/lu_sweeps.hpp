@@ -5,8 +5,11 @@
 // rows it reaches.  A column's entries are read from LDS one block of steps ahead of the
 // block in work (the compiler left to itself reads one step ahead and waits for LDS at every
 // step: about 105 cycles a step), and the entries of rows that a column does not reach are
-// replaced by zero ahead of the chain, so that no select stands in it.  FP64, one color of the
-// fused step (k_patch.hip): 8^3 11.6 -> 9.2 us, 16^3 17.7 -> 15.8 us, the same results bit for bit.
+// replaced by zero ahead of the chain, so that no select stands in it (putting every unknown aside
+// at its step instead costs 3 % of a color).  FP64, one color of the fused step (k_patch.hip): 8^3
+// 11.6 -> 9.2 us, 16^3 17.7 -> 15.8 us, the same results bit for bit.
+// An unknown that is not finite would come to the rows that its column does not reach as zero
+// times it.  Its own row shows it at the end; the sweep is then run again with selects.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -43,6 +46,12 @@ struct Ld<float, uint16_t> {
   }
 };
 
+// some unknown of the patch is not finite (row 64 + lane exists on the first 21 lanes)
+template <typename T>
+__device__ __forceinline__ bool any_not_finite(int lane, T x0, T x1) {
+  return __any(!(fabs(x0) < T(INFINITY)) || (lane < NLOC - 64 && !(fabs(x1) < T(INFINITY))));
+}
+
 constexpr int LU_STEPS = 6;   // steps of a block; two blocks of entries are in registers
 
 // x := L^{-1} x; s: the packed L part in LDS, L(r, k) at lu_loff(k) + r - k - 1, with 64 readable
@@ -51,6 +60,7 @@ template <typename T, typename F>
 __device__ __forceinline__ void lower_sweep(const F *s, int lane, T &x0, T &x1) {
   constexpr int N = NLOC - 1, NB = (N + LU_STEPS - 1) / LU_STEPS;
   const F *const sl0 = s + lane, *const sl1 = sl0 + 64;
+  const T r0 = x0, r1 = x1;
   T a[2][LU_STEPS], b[2][LU_STEPS];
   auto fetch = [&](int blk, T (&p)[LU_STEPS], T (&q)[LU_STEPS]) {
 #pragma unroll
@@ -84,6 +94,16 @@ __device__ __forceinline__ void lower_sweep(const F *s, int lane, T &x0, T &x1) 
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  if (!any_not_finite(lane, x0, x1)) return;
+  x0 = r0;
+  x1 = r1;
+#pragma unroll 1
+  for (int k = 0; k < N; ++k) {
+    const int o = lu_loff(k) - k - 1;
+    const T xk = k < 64 ? bcast(x0, k) : bcast(x1, k - 64);
+    if (lane > k) x0 = tfma(-xk, Ld<T, F>::get(sl0, o), x0);
+    if (lane + 64 > k) x1 = tfma(-xk, Ld<T, F>::get(sl1, o), x1);
+  }
 }
 
 // x := U^{-1} x; s: the packed U part, U(r, k) at lu_uoff(k) + r.  A row's value is final once its
@@ -95,6 +115,7 @@ template <typename T, typename F>
 __device__ __forceinline__ void upper_sweep(const F *s, int lane, bool two, T &x0, T &x1) {
   constexpr int NB = (NLOC + LU_STEPS - 1) / LU_STEPS;
   const F *const sl0 = s + lane, *const sl1 = sl0 + 64;
+  const T r0 = x0, r1 = x1;
   const T dg0 = Ld<T, F>::get(s, lu_uoff(lane) + lane);
   const T dg1 = two ? Ld<T, F>::get(s, lu_uoff(64 + lane) + 64 + lane) : T(1);
   const T rc0 = T(1) / dg0, rc1 = T(1) / dg1;
@@ -138,6 +159,19 @@ __device__ __forceinline__ void upper_sweep(const F *s, int lane, bool two, T &x
   }
   x0 = quotient(x0, dg0, rc0);
   x1 = quotient(x1, dg1, rc1);
+  if (!any_not_finite(lane, x0, x1)) return;
+  x0 = r0;
+  x1 = r1;
+#pragma unroll 1
+  for (int k = NLOC - 1; k >= 0; --k) {
+    const int o = lu_uoff(k);
+    const T q0 = quotient(x0, dg0, rc0), q1 = quotient(x1, dg1, rc1);
+    const T xk = k < 64 ? bcast(q0, k) : bcast(q1, k - 64);
+    if (lane == k) x0 = q0;
+    if (lane + 64 == k) x1 = q1;
+    if (lane < k) x0 = tfma(-xk, Ld<T, F>::get(sl0, o), x0);
+    if (lane + 64 < k) x1 = tfma(-xk, Ld<T, F>::get(sl1, o), x1);
+  }
 }
 
 }  // namespace pmg
