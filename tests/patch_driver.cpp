@@ -82,6 +82,18 @@ static void records(const Sys &S, const PatchTables &T, int nc, const int *ptr, 
         CHECK(rc[PR_RUN + i / 4] >= 0 && rc[PR_RUN + i / 4] + i % 4 < d.n_pdof);
         hp[i] = p[rc[PR_RUN + i / 4] + i % 4];
       }
+      // places of a quad's A (B) rows without an entry read the zero behind the halo
+      for (int qd = 0; qd < 8; ++qd) {
+        const int off = fp64 ? (T.grid ? PatchShape64<true>::off_a(qd) : PatchShape64<false>::off_a(qd))
+                             : 64 * (T.grid ? PatchShape<true>::off_a(qd) : PatchShape<false>::off_a(qd));
+        const int len = fp64 ? 128 * (T.grid ? PatchShape64<true>::a(qd) : PatchShape64<false>::a(qd))
+                             : 64 * (((T.grid ? PatchShape<true>::a(qd) : PatchShape<false>::a(qd)) + 1) / 2);
+        int entries = 0, used = 0;
+        for (int e = 4 * qd; e < 4 * qd + 4; ++e) entries += rc[PR_DESC + 4 * e + 2] & 255;
+        for (int w = off; w < off + len; ++w)
+          used += ((pat[w] & 0xffffu) != unsigned(PT_ZERO)) + ((pat[w] >> 16) != unsigned(PT_ZERO));
+        CHECK(used == entries);
+      }
       for (int e = 0; e < 32; ++e) {
         const int *dc = rc + PR_DESC + 4 * e, qd = e / 4;
         const int n = dc[2] & 255, m = (dc[2] >> 8) & 255, row = (dc[2] >> 16) & 255;

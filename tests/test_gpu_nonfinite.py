@@ -3,7 +3,9 @@
 The local and coarse solves in FP64 have the same finite and non-finite unknowns as the oracle's
 dgetrs, which leaves an unknown that is finished alone: right-hand sides of about 1e306 let some
 of the unknowns of a patch (of a block of 64 of the coarse system) overflow, after the pressures
-and some velocities have come out finite."""
+and some velocities have come out finite.  In the FP32 color step an infinite velocity reaches the
+rows that are coupled to it and no others: in a patch where it stands in one row, the product with
+the stored inverse is infinite, not the NaN of two infinities or of zero times infinity."""
 import numpy as np
 import pytest
 
@@ -62,3 +64,31 @@ def test_finished_unknowns_of_a_coarse_block_stay(box, faces, e):
     y = mg.solve_exact(f)
     mg.close()
     assert np.array_equal(np.isfinite(y[free]), np.isfinite(x[free]))
+
+
+@pytest.mark.parametrize("precision", [1, 2])
+def test_uncoupled_rows_stay(precision):
+    from to_merge_master_parmoon_amd.multigrid import build_hierarchy, color_cells
+    prob = _problem((4, 4, 4), 63)
+    d, a = prob.descs[1], prob.arrays(1)
+    rp, kc, bp, bc = a["a_rowptr"], a["a_kcol"], a["b_rowptr"], a["b_kcol"]
+    ug, pg = a["u_global"].reshape(-1, 27), a["p_global"].reshape(-1, 4)
+    _, ptr, order = color_cells(d.n_cells, a["u_global"], d.n_udof)
+    # cells of the first color whose lowest dof stands in one row only, an active vertex row of
+    # another number of entries than 16 k (the lanes past its end read no entry)
+    cells = []
+    for c in order[:ptr[1]]:
+        rows = [kc[rp[r]:rp[r + 1]] for r in ug[c]]
+        g = min(r.min() for r in rows)
+        inside = [r for r, cols in zip(ug[c], rows) if g in cols]
+        if g < d.n_active and len(inside) == 1 and inside[0] < d.n_active and (rp[inside[0] + 1] - rp[inside[0]]) % 16 \
+                and not any(g in bc[bp[i]:bp[i + 1]] for i in pg[c]):
+            cells.append((c, g))
+    assert cells
+    mg = build_hierarchy(prob, params(precision=precision))
+    c, g = cells[0]
+    u = np.zeros(mg.n_dof[1])
+    u[g] = np.inf
+    y = mg.cell_vanka(1, u, np.zeros_like(u), 1)
+    mg.close()
+    assert np.isinf(y[3 * d.n_udof + pg[c]]).all()

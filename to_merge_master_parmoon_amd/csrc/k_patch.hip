@@ -216,7 +216,7 @@ struct VelRow9<SH, 1> {
 
 template <typename F, bool FULL>
 struct PatchLds {
-  float4 hv[PT_HALO];
+  float4 hv[PT_HALO + 1];                   // the halo, and zeros at PT_ZERO
   float hp[4 * PT_RUNS];
   float rs[RLOC_STRIDE], xs[RLOC_STRIDE];   // local residual and solution
   float M[FULL ? 4 : SCH_STRIDE];           // stored block form
@@ -304,8 +304,10 @@ __device__ __forceinline__ void patch_wave(const PatchStep &P, const F *__restri
     S.hv[t + 256] = h1;
     S.hp[t] = hq;
   }
-  if constexpr (W == 3)
+  if constexpr (W == 3) {
     if (l64 < RLOC_STRIDE - NLOC) S.rs[NLOC + l64] = 0.0f;
+    if (l64 == 63) S.hv[PT_ZERO] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
   patch_barrier();
   A.residual(S.hv, S.hp, S.rs, l64);
   B.residual(S.hv, S.hp, S.rs, l64);
@@ -451,6 +453,10 @@ __device__ __forceinline__ double *velocity_at(const PatchStep64 &P, int loc) {
   return p;
 }
 
+// between the components of the halo in LDS (PT_ZERO behind it; a multiple of 64, so that one
+// instruction reads two components)
+constexpr int HSTRIDE = PT_HALO + 64;
+
 // four consecutive entries from p on (8-byte aligned)
 __device__ __forceinline__ void ld4d(const double *p, double (&o)[4]) { ld4(p, o); }
 __device__ __forceinline__ int window(int jb, int n) { return n >= 4 ? min(jb, n - 4) : 0; }
@@ -504,7 +510,7 @@ struct Row64 {
       for (int u = 0; u < 4; ++u) {
         const double *y = hv + at(ib, u);
         const bool ok = own(4 * lane, n, u);
-        const double z1 = ok ? y[0] : 0.0, z2 = ok ? y[PT_HALO] : 0.0, z3 = ok ? y[2 * PT_HALO] : 0.0;
+        const double z1 = ok ? y[0] : 0.0, z2 = ok ? y[HSTRIDE] : 0.0, z3 = ok ? y[2 * HSTRIDE] : 0.0;
         // contracted as row_b_v is compiled in k_vanka_res
         s += fma(b[2][u], z3, u == 0 ? fma(b[1][u], z2, b[0][u] * z1) : fma(b[0][u], z1, b[1][u] * z2));
       }
@@ -519,8 +525,8 @@ struct Row64 {
           const double *y = hv + at(ia[k], u);
           const double w = own(64 * k + 4 * lane, n, u) ? a[k][u] : 0.0;
           s1 += w * y[0];
-          s2 += w * y[PT_HALO];
-          s3 += w * y[2 * PT_HALO];
+          s2 += w * y[HSTRIDE];
+          s3 += w * y[2 * HSTRIDE];
         }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -538,7 +544,7 @@ struct Row64 {
 };
 
 struct Patch64Lds {
-  double hv[3 * PT_HALO], hp[4 * PT_RUNS], rs[RLOC_STRIDE];
+  double hv[3 * HSTRIDE], hp[4 * PT_RUNS], rs[RLOC_STRIDE];
   v4u fac[32 + 64 * 29];   // a factor part after 64 entries of padding (k_vanka_solve)
 };
 
@@ -602,12 +608,14 @@ __device__ __forceinline__ void patch_wave64(const PatchStep64 &P, long pos, int
 #pragma unroll
   for (int q = 0; q < NU; ++q) rU[q] = gU[l64 + 64 * (4 * q + W)];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) S.hv[c * PT_HALO + t] = h0[c];
+  for (int c = 0; c < 3; ++c) S.hv[c * HSTRIDE + t] = h0[c];
   if constexpr (W < 2) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) S.hv[c * PT_HALO + t + 256] = h1[c];
+    for (int c = 0; c < 3; ++c) S.hv[c * HSTRIDE + t + 256] = h1[c];
     S.hp[t] = hq;
   }
+  if constexpr (W == 3)
+    if (l64 < 3) S.hv[l64 * HSTRIDE + PT_ZERO] = 0.0;
   patch_barrier();
   A.residual(S.hv, S.hp, S.rs, l64);
   B.residual(S.hv, S.hp, S.rs, l64);
@@ -629,10 +637,10 @@ __device__ __forceinline__ void patch_wave64(const PatchStep64 &P, long pos, int
   patch_barrier();
   if constexpr (W == 0) {
     upper_sweep<double, double>(fac, l64, two, x0, x1);
-    velocity_at(P, out0)[long(c0) * P.N] = S.hv[c0 * PT_HALO + own0] + P.damp * x0;
+    velocity_at(P, out0)[long(c0) * P.N] = S.hv[c0 * HSTRIDE + own0] + P.damp * x0;
     if (two) {
       if (j1 < NU_LOC)
-        velocity_at(P, out1)[2L * P.N] = S.hv[2 * PT_HALO + own1] + P.damp * x1;
+        velocity_at(P, out1)[2L * P.N] = S.hv[2 * HSTRIDE + own1] + P.damp * x1;
       else
         P.u[3L * P.N + out1] = v1 + P.damp * x1;
     }

@@ -110,8 +110,9 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
       T.grid = T.grid && len_a(u[j]) <= 16 * G::a(qd) && len_bt(u[j]) <= 16 * G::bt(qd);
     }
   }
-  int off_a[8], off_bt[8];   // words
+  int off_a[8], off_bt[8], len_pat[8];   // words
   for (int qd = 0; qd < 8; ++qd) {
+    len_pat[qd] = fp64 ? 128 * (T.grid ? G64::a(qd) : R64::a(qd)) : 64 * (((T.grid ? G::a(qd) : R::a(qd)) + 1) / 2);
     off_a[qd] = fp64 ? (T.grid ? G64::off_a(qd) : R64::off_a(qd)) : 64 * (T.grid ? G::off_a(qd) : R::off_a(qd));
     off_bt[qd] = fp64 ? (T.grid ? G64::off_bt(qd) : R64::off_bt(qd)) : 64 * (T.grid ? G::off_bt(qd) : R::off_bt(qd));
   }
@@ -201,14 +202,19 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
         // rows and their column positions
         for (int e = 0; e < 32; ++e) rc[PR_DESC + 4 * e + 2] = PT_NOROW << 16;
         W.pat.assign(words, 0u);
+        for (int qd = 0; qd < 8; ++qd)
+          std::fill(W.pat.begin() + off_a[qd], W.pat.begin() + off_a[qd] + len_pat[qd], uint32_t(PT_ZERO) * 0x10001u);
+        auto set = [&](size_t w, int half, int pos) {
+          W.pat[w] = (W.pat[w] & ~(0xffffu << (16 * half))) | uint32_t(pos) << (16 * half);
+        };
         auto put = [&](int off, int e, int j, int n, int pos) {   // entry j of n of the row at place e
           if (fp64) {
             // entry u of the lane's window, which starts at most n - 4 (row_window)
             const int lane = j % 64 / 4, jb = j / 4 * 4, first = n >= 4 ? std::min(jb, n - 4) : 0, u = j - first;
-            W.pat[size_t(off) + 2 * (64 * (j / 64) + (e % 4) * 16 + lane) + u / 2] |= uint32_t(pos) << (16 * (u & 1));
+            set(size_t(off) + 2 * (64 * (j / 64) + (e % 4) * 16 + lane) + u / 2, u & 1, pos);
           } else {
             const int step = j / 16, lane = (e % 4) * 16 + j % 16;
-            W.pat[size_t(off) + 64 * (step / 2) + lane] |= uint32_t(pos) << (16 * (step & 1));
+            set(size_t(off) + 64 * (step / 2) + lane, step & 1, pos);
           }
         };
         auto desc = [&](int e, int k0, int q0b, int n, int m, int row, int g) {
@@ -229,7 +235,7 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
             const int c = d->bt_kcol[q0b + k];
             put(off_bt[qd], e, k, m, 4 * W.pmark[c / 4] + c % 4);
           }
-          W.pat[own + j / 2] |= uint32_t(W.mark[g]) << (16 * (j & 1));
+          set(size_t(own) + j / 2, j & 1, W.mark[g]);
         }
         for (int j = 0; j < NP; ++j) {
           const int e = 4 + j, k0 = d->b_rowptr[p[j]], n = d->b_rowptr[p[j] + 1] - k0;

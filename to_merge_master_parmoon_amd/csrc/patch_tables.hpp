@@ -13,6 +13,7 @@
 namespace pmg {
 
 constexpr int PT_HALO = 384;    // most velocity dofs in a patch's halo (343 on a hexahedral grid)
+constexpr int PT_ZERO = PT_HALO; // halo position that holds zero: what lanes past a row's end read
 constexpr int PT_RUNS = 32;     // most runs of four pressure dofs in a halo (27 there)
 constexpr int PT_ROW = 128;     // longest A row, 8 steps of 16 lanes
 constexpr int PT_BT = 32;       // longest BT row and B row, 2 steps
@@ -35,7 +36,8 @@ constexpr int PT_NOROW = 255;   // row number of an empty place
 // A pattern holds the positions of the rows' columns in the halo, shared by all cells whose rows
 // have the same structure (a few hundred on a refined mesh): 32-bit words of two 16-bit
 // positions, steps 2 p and 2 p + 1 of a lane at (off_a(quad) + p) * 64 + lane (off_bt for the
-// BT row); then the patch's own 27 dofs.
+// BT row); then the patch's own 27 dofs.  Places without an entry hold PT_ZERO (A, B) or 0 (BT,
+// whose values the kernels mask), so that no row is touched by a value it is not coupled to.
 template <bool GRID>
 struct PatchShape {
   static constexpr int a(int quad) { return quad == 1 ? 2 : !GRID ? 8 : quad == 0 || quad == 2 ? 8 : quad == 3 || quad == 7 ? 3 : 5; }
