@@ -555,6 +555,33 @@ __global__ __launch_bounds__(TRSM_BIG_T) void k_trsm_big(const double *__restric
   }
 }
 
+// *info = -1 if the smallest pivot of the factored lu (n x n) is below PIVOT_RANGE_MIN times the
+// largest and no pivot was zero.  The inverse of a block loses about as many digits as its pivots
+// range over, which a pivoted LU of the whole system need not: 1.1e-16 / 1e-9 is the rounding of
+// the FP32 vectors that the solution goes to.
+constexpr double PIVOT_RANGE_MIN = 1e-9;
+__global__ __launch_bounds__(256) void k_pivot_range(const double *__restrict__ lu, int n, int ld, int *__restrict__ info) {
+  __shared__ double lo[256], hi[256];
+  const int t = threadIdx.x;
+  double a = INFINITY, b = 0.0;
+  for (int i = t; i < n; i += 256) {
+    const double p = fabs(lu[long(i) * ld + i]);
+    a = fmin(a, p);
+    b = fmax(b, p);
+  }
+  lo[t] = a;
+  hi[t] = b;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (t < o) {
+      lo[t] = fmin(lo[t], lo[t + o]);
+      hi[t] = fmax(hi[t], hi[t + o]);
+    }
+    __syncthreads();
+  }
+  if (t == 0 && *info == 0 && lo[0] < PIVOT_RANGE_MIN * hi[0]) *info = -1;
+}
+
 // ------------------------------------------------------------------ FP64 GEMM
 // C = alpha A B + beta C (row-major; A M x K, B K x N); one wavefront per 16 x 16 tile of C,
 // four per workgroup, K in steps of 4 on the matrix cores.
@@ -688,6 +715,8 @@ void coarse_block_factor(CoarseBlock &B, hipStream_t s) {
   const int slabs = (ldx + TRSM_NR - 1) / TRSM_NR;
   if (coarse_block_panels(m)) {
     lu_factor_panels(B.A, m, B.ipiv, B.sigA, B.ubuf, B.swp, B.info, s);
+    k_pivot_range<<<1, 256, 0, s>>>(B.A, m, m, B.info);
+    PMG_HIP_CHECK(hipGetLastError());
     k_trsm_big<<<slabs, TRSM_BIG_T, 0, s>>>(B.A, m, m, B.sigA, B.X, ldx, ldx, B.X, ldx);
   } else {
     k_lu_wg<<<1, LU_T, 0, s>>>(B.A, m, m, B.sigA, B.info);
@@ -703,6 +732,10 @@ void coarse_block_factor(CoarseBlock &B, hipStream_t s) {
   // S = P^T L U; S^{-1} into the last q columns of P1; -Q = -S^{-1} V into the first 3m
   k_lu_wg<<<1, LU_T, 0, s>>>(B.S, q, q, B.sigS, B.info + 1);
   PMG_HIP_CHECK(hipGetLastError());
+  if (coarse_block_panels(m)) {
+    k_pivot_range<<<1, 256, 0, s>>>(B.S, q, q, B.info + 1);
+    PMG_HIP_CHECK(hipGetLastError());
+  }
   k_trsm_wg<<<(q + TRSM_NR - 1) / TRSM_NR, TRSM_T, 0, s>>>(B.S, q, q, B.sigS, nullptr, 0, q, B.P1 + 3L * m, ldp);
   PMG_HIP_CHECK(hipGetLastError());
   gemm(q, 3 * m, q, -1.0, B.P1 + 3L * m, ldp, B.V, 3 * m, 0.0, B.P1, ldp, s);

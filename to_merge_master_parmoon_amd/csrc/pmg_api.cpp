@@ -382,13 +382,18 @@ std::vector<int> build_patch_map(const pmg_level_desc *d, const std::vector<int>
 // and its time, and the wait-bound flag of the coarse triangular sweeps.
 void check_coarse(pmg_ctx *c, Coarse &C);
 void check_nodal(pmg_ctx *c);
+void settle_coarse(pmg_ctx *c, const DevLevel &D, Coarse &C);
 void check_deferred(pmg_ctx *c) {
   if (!c->batch) {
+    if (!c->L.empty()) settle_coarse(c, c->L[0], c->coarse);
     check_coarse(c, c->coarse);
     check_nodal(c);
     return;
   }
-  for (auto &b : c->bi) check_coarse(c, b.co);
+  for (auto &b : c->bi) {
+    settle_coarse(c, b.cl, b.co);
+    check_coarse(c, b.co);
+  }
 }
 // nodal Vanka: the largest pressure dof (+1) whose local system had a zero pivot in the
 // sweeps since the last check; reported once and cleared (the stream is idle here)
@@ -845,10 +850,7 @@ double coarse_visit_flops(const Coarse &C) {
 // coarse solve in FP64 (vectors of type T converted at the boundary)
 template <typename T>
 void coarse_solve_t(pmg_ctx *c, const DevLevel &D, T *u, const T *f) {
-  if (c->coarse.pending) {
-    PMG_HIP_CHECK(hipStreamWaitEvent(c->stream, c->coarse.ev_done, 0));
-    c->coarse.pending = false;
-  }
+  settle_coarse(c, D, c->coarse);
   Timed tm(c, &c->tm.coarse_solve, coarse_visit_bytes(c->coarse), coarse_visit_flops(c->coarse));
   if constexpr (sizeof(T) == 8) {
     coarse_solve_any(c->coarse, D.op64(), f, u, c->stream);
@@ -898,14 +900,11 @@ void build_cb_jobs(pmg_ctx *c) {
 // the block-form ones in one batched visit (three launches), the others one by one
 template <typename T>
 void batch_coarse(pmg_ctx *c, const DevLevel &D, T *u, const T *f) {
+  for (int k : D.coarse_insts) settle_coarse(c, c->bi[k].cl, c->bi[k].co);
   if (D.n_cb_jobs > 0) {
     double by = 0.0, fl = 0.0;
     for (int k : D.cb_job_prob) {
       BatchProblem &b = c->bi[k];
-      if (b.co.pending) {
-        PMG_HIP_CHECK(hipStreamWaitEvent(c->stream, b.co.ev_done, 0));
-        b.co.pending = false;
-      }
       by += coarse_visit_bytes(b.co);
       fl += coarse_visit_flops(b.co);
     }
@@ -917,10 +916,6 @@ void batch_coarse(pmg_ctx *c, const DevLevel &D, T *u, const T *f) {
     if (!c->b_live.empty() && !c->b_live[k]) continue;   // finished: left out, its result is unused
     BatchProblem &b = c->bi[k];
     if (b.in_job) continue;
-    if (b.co.pending) {
-      PMG_HIP_CHECK(hipStreamWaitEvent(c->stream, b.co.ev_done, 0));
-      b.co.pending = false;
-    }
     Timed tm(c, &c->tm.coarse_solve, coarse_visit_bytes(b.co), coarse_visit_flops(b.co));
     launch_gather_d<T>(b.cf, f, b.cidx, b.n_dof_coarse, c->stream);
     coarse_solve_any(b.co, b.cl.op64(), b.cf, b.cu, c->stream);
@@ -1024,13 +1019,8 @@ void cycle(pmg_ctx *c, int i, bool zero) {
 
 // the main stream waits for coarse factorizations still running on the second stream
 void resolve_pending(pmg_ctx *c) {
-  auto wait = [&](Coarse &C) {
-    if (!C.pending) return;
-    PMG_HIP_CHECK(hipStreamWaitEvent(c->stream, C.ev_done, 0));
-    C.pending = false;
-  };
-  wait(c->coarse);
-  for (auto &b : c->bi) wait(b.co);
+  settle_coarse(c, c->L[0], c->coarse);
+  for (auto &b : c->bi) settle_coarse(c, b.cl, b.co);
 }
 bool coarse_pending(const pmg_ctx *c) {
   if (c->coarse.pending) return true;
@@ -1180,9 +1170,9 @@ void coarse_block_alloc(pmg_ctx *c, CoarseBlock &B, int m, int q) {
 // block form when the smoother runs in mixed precision on the shared velocity block
 // (FP64 inverses of the blocks, each visit two matrix-vector phases), otherwise as one
 // dense LU whose factors equal dgetf2's (the FP64 form, parity with SolveExact)
-void start_coarse_factor(pmg_ctx *c, const DevLevel &D, Coarse &C, int pin) {
+void start_coarse_factor(pmg_ctx *c, const DevLevel &D, Coarse &C, int pin, bool dense = false) {
   const int m = D.n_active, q = D.n_pdof - pin;
-  const bool block = mixed(c) && D.a_shared && coarse_block_fits(m, q);
+  const bool block = !dense && mixed(c) && D.a_shared && coarse_block_fits(m, q);
   if (block) {
     if (!C.ev_start) {
       PMG_HIP_CHECK(hipEventCreate(&C.ev_start));
@@ -1205,6 +1195,10 @@ void start_coarse_factor(pmg_ctx *c, const DevLevel &D, Coarse &C, int pin) {
     PMG_HIP_CHECK(hipMemsetAsync(C.info, 0, sizeof(int), c->stream2));
     launch_cb_build(D, C.cb, c->stream2);
     coarse_block_factor(C.cb, c->stream2);
+    if (coarse_block_panels(m)) {
+      if (!C.h_info) PMG_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&C.h_info), 2 * sizeof(int)));
+      PMG_HIP_CHECK(hipMemcpyAsync(C.h_info, C.cb.info, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream2));
+    }
   } else {
     launch_coarse_build(D, C, c->stream2);
     coarse_lu_factor(C, c->stream2);
@@ -1212,6 +1206,24 @@ void start_coarse_factor(pmg_ctx *c, const DevLevel &D, Coarse &C, int pin) {
   PMG_HIP_CHECK(hipEventRecord(C.ev_done, c->stream2));
   C.pending = true;
   C.info_pending = true;
+}
+
+// The main stream waits for a factorization that still runs on the second stream (never inside
+// a capture: the first cycle after a set-up is eager).  The block form needs a velocity block
+// that can be inverted by itself, the dense LU pivots over the whole system: above 512 velocity
+// unknowns the host looks at the pivots of the blocks first, and a system whose blocks have a
+// pivot that is zero or too small (k_pivot_range) is factored as a whole.
+void settle_coarse(pmg_ctx *c, const DevLevel &D, Coarse &C) {
+  if (!C.pending) return;
+  if (C.block && coarse_block_panels(C.cb.m)) {
+    PMG_HIP_CHECK(hipEventSynchronize(C.ev_done));
+    if (C.h_info[0] || C.h_info[1]) {
+      start_coarse_factor(c, D, C, C.pin, true);
+      if (c->batch) build_cb_jobs(c);
+    }
+  }
+  PMG_HIP_CHECK(hipStreamWaitEvent(c->stream, C.ev_done, 0));
+  C.pending = false;
 }
 
 void setup_factors(pmg_ctx *c) {
@@ -1979,7 +1991,9 @@ int pmg_ctx_destroy(pmg_ctx *c) {
   if (c->evs) (void)hipEventDestroy(c->evs);
   if (c->coarse.ev_start) (void)hipEventDestroy(c->coarse.ev_start);
   if (c->coarse.ev_done) (void)hipEventDestroy(c->coarse.ev_done);
+  if (c->coarse.h_info) (void)hipHostFree(c->coarse.h_info);
   for (auto &b : c->bi) {
+    if (b.co.h_info) (void)hipHostFree(b.co.h_info);
     if (b.co.ev_start) (void)hipEventDestroy(b.co.ev_start);
     if (b.co.ev_done) (void)hipEventDestroy(b.co.ev_done);
   }

@@ -313,6 +313,7 @@ struct Coarse {
   unsigned *sync = nullptr;
   unsigned long long *words = nullptr;
   int *err = nullptr;   // set by a wait past its limit
+  int *h_info = nullptr;   // (coarse_block_panels) the block form's pivot flags, pinned host memory
   // the factorization runs on the second stream; the main stream waits for ev_done only
   // before the first coarse solve, and the pivot check happens at the next host sync
   hipEvent_t ev_start = nullptr, ev_done = nullptr;
@@ -466,7 +467,7 @@ void launch_coarse_rhs(const OpView<double> &op, const double *f, const int *sig
 // (asynchronous; cb.info gets the zero-pivot flags of the two LUs) and one visit from the
 // reduced right-hand side rr into the level vector u
 bool coarse_block_fits(int m, int q);
-bool coarse_block_panels(int m);   // A is factored by lu_factor_panels (info[0] gets its zero-pivot flag)
+bool coarse_block_panels(int m);   // A is factored by lu_factor_panels (info[0]: its zero-pivot flag, -1 for a small one)
 void lu_factor_panels(double *a, int n, int *ipiv, int *sigma, double *ubuf, int *swp, int *info, hipStream_t s);
 void launch_cb_build(const DevLevel &L, CoarseBlock &B, hipStream_t s);
 void coarse_block_factor(CoarseBlock &B, hipStream_t s);
