@@ -770,11 +770,19 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   }
 }
 
-// the buffer of the FP64 operator's interleaved input velocity, for the largest level
+// With the shared velocity block the FP64 operator gathers an interleaved copy of its input's
+// velocity where that pays for the pass that makes it (3 x 8 B read, 4 x 8 B written per dof):
+// pmg_defect at 32^3 (274,625 velocity dofs) 198 -> 188 us, at 24^3 (117,649) 89 -> 90 us.  The
+// matvec of FGMRES without and with the copy: 35,937 dofs 23.4, 26.2 us; 68,921 40.3, 43.2;
+// 117,649 72.7, 73.9; pmg_matvec at 207,025 124, 122, at 274,625 171, 160
+constexpr int XA_MIN_UDOF = 150000;
+bool takes_xa(const pmg_ctx *c, const DevLevel &D) { return !c->batch && D.a_shared && D.n_udof >= XA_MIN_UDOF; }
+// the buffer of that copy, for the largest level that takes it
 void ensure_xa(pmg_ctx *c) {
   long n = 0;
-  for (const auto &D : c->L) n = std::max<long>(n, D.n_udof);
-  if (c->batch || c->xa64_n >= n) return;
+  for (const auto &D : c->L)
+    if (takes_xa(c, D)) n = std::max<long>(n, D.n_udof);
+  if (c->xa64_n >= n) return;
   drop_graph(c);   // a captured V-cycle may hold the old buffer
   dfree(c, c->xa64);
   c->xa64 = nullptr;
@@ -782,13 +790,9 @@ void ensure_xa(pmg_ctx *c) {
   c->xa64 = dalloc<double>(c, 4 * size_t(n));
   c->xa64_n = n;
 }
-// With the shared velocity block the FP64 operator gathers an interleaved copy of its input's
-// velocity where that pays for the pass that makes it (3 x 8 B read, 4 x 8 B written per dof):
-// pmg_defect at 32^3 (274,625 velocity dofs) 198 -> 188 us, at 24^3 (117,649) 89 -> 90 us
-constexpr int XA_MIN_UDOF = 150000;
 OpView<double> op64_for(pmg_ctx *c, const DevLevel &D, const double *x) {
   OpView<double> o = D.op64();
-  if (D.a_shared && c->xa64_n >= D.n_udof && D.n_udof >= XA_MIN_UDOF) {
+  if (takes_xa(c, D) && c->xa64_n >= D.n_udof) {
     launch_interleave3(c->xa64, x, D.n_udof, c->stream);
     o.xa = c->xa64;
   }
