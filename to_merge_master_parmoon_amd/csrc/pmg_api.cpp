@@ -53,7 +53,7 @@ struct pmg_ctx {
   // FGMRES workspace
   int restart_alloc = 0;
   double *V = nullptr, *Z = nullptr, *W = nullptr, *Hdev = nullptr, *coef = nullptr;
-  // the FGMRES operator's input velocity interleaved (4 doubles per finest velocity dof)
+  // the FP64 operator's input velocity interleaved (4 doubles per dof, of the largest level that takes it)
   double *xa64 = nullptr;
   long xa64_n = 0;
   double *hpin = nullptr;   // pinned host scalars
@@ -612,6 +612,65 @@ void nodal_sweep(pmg_ctx *c, DevLevel &D, double *u, const double *f, double *au
   }
   launch_relax<double>(u, aux, alpha, D.n_dof, c->stream);
   if (last) set_dirichlet(c, D, u, f);
+}
+
+// The level's present form is one that the fused color step has (k_patch.hip): FP64 with the shared
+// velocity block, the stored inverses without refinement steps.  Records and copies of the
+// velocity are built for such levels only, 2.3 KB a cell and up to three velocities; a level that
+// turns to such a form later gets them at its set-up.
+bool takes_patch_step(const pmg_ctx *c, const DevLevel &D) {
+  if (D.lu) return D.a_shared;
+  return (D.minv32 || D.minv16) && c->prm.bf16_refine_steps == 0;
+}
+// ug, pg: dofs of every cell; order: the cells in color order.  A level that fits no record keeps
+// the two launches.
+void build_patch_records(pmg_ctx *c, DevLevel &D, const pmg_level_desc *d, const std::vector<int> &ug,
+                         const std::vector<int> &pg, const int *order) {
+  D.patch_tried = true;
+  PatchTables T;
+  build_patch_tables(d, ug, pg, D.n_colors, D.ptr_colors.data(), order, D.lu != nullptr, T);
+  if (!T.ok) return;
+  drop_graph(c);   // a captured V-cycle holds the two launches and the old copy
+  int *rec = dalloc<int>(c, T.rec.size());
+  h2d(c, rec, T.rec.data(), T.rec.size());
+  D.patch_pat = dalloc<uint32_t>(c, T.pat.size());
+  h2d(c, D.patch_pat, T.pat.data(), T.pat.size());
+  D.patch_stride = T.stride;
+  D.patch_grid = T.grid;
+  if (D.lu) {
+    D.patch_alt = dalloc<double>(c, 3 * size_t(D.n_udof) * std::max(1, T.n_buffers - 1));
+  } else if (T.n_buffers > 1) {
+    float *ua = dalloc<float>(c, 4 * size_t(D.n_udof) * T.n_buffers);
+    dfree(c, D.ua32);
+    D.ua32 = ua;
+  }
+  PMG_HIP_CHECK(hipStreamSynchronize(c->stream));
+  D.patch_rec = rec;
+}
+// the same from the level's own arrays
+void build_patch_records(pmg_ctx *c, DevLevel &D, const std::vector<int> &ug, const std::vector<int> &pg) {
+  auto get = [&](const int *p, size_t n) {
+    std::vector<int> v(n);
+    PMG_HIP_CHECK(hipMemcpyAsync(v.data(), p, n * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    PMG_HIP_CHECK(hipStreamSynchronize(c->stream));
+    return v;
+  };
+  const std::vector<int> ar = get(D.a_rowptr, D.n_udof + 1), ac = get(D.a_kcol, D.a_nnz);
+  const std::vector<int> br = get(D.b_rowptr, D.n_pdof + 1), bc = get(D.b_kcol, D.b_nnz);
+  const std::vector<int> tr = get(D.bt_rowptr, D.n_udof + 1), tc = get(D.bt_kcol, D.bt_nnz);
+  const std::vector<int> order = get(D.cell_reorder, D.n_cells);
+  pmg_level_desc d{};
+  d.n_cells = D.n_cells;
+  d.n_udof = D.n_udof;
+  d.n_active = D.n_active;
+  d.n_pdof = D.n_pdof;
+  d.a_rowptr = ar.data();
+  d.a_kcol = ac.data();
+  d.b_rowptr = br.data();
+  d.b_kcol = bc.data();
+  d.bt_rowptr = tr.data();
+  d.bt_kcol = tc.data();
+  build_patch_records(c, D, &d, ug, pg, order.data());
 }
 
 // the FP32 sweep with nine velocity blocks in one launch per color (k_patch.hip)
@@ -1261,6 +1320,7 @@ void setup_factors(pmg_ctx *c) {
     DevLevel &D = c->L[l];
     if (D.factors_ready) continue;
     const hipStream_t ps = c->stream;
+    if (!D.patch_tried && takes_patch_step(c, D)) build_patch_records(c, D, c->h_u_global[l], c->h_p_global[l]);
     if (D.nodal) {   // nodal Vanka assembles and solves its patches at every visit
       D.factors_ready = true;
       continue;
@@ -2304,24 +2364,9 @@ static int add_level(pmg_ctx *c, const pmg_level_desc *d, int *level_out, bool m
         D.minv16 = dalloc<uint16_t>(c, minvn);
         launch_fill<uint16_t>(D.minv16, uint16_t(0), long(minvn), c->stream);
       }
+      if (D.minv32 || D.minv16) D.ua32 = dalloc<float>(c, 4 * size_t(D.n_udof));
       if (D.lu || D.minv32 || D.minv16) {
-        PatchTables T;
-        build_patch_tables(d, ug, pg, nc, D.ptr_colors.data(), reo.data(), D.lu != nullptr, T);
-        if (T.ok) {
-          D.patch_rec = dalloc<int>(c, T.rec.size());
-          h2d(c, D.patch_rec, T.rec.data(), T.rec.size());
-          D.patch_pat = dalloc<uint32_t>(c, T.pat.size());
-          h2d(c, D.patch_pat, T.pat.data(), T.pat.size());
-          D.patch_stride = T.stride;
-          D.patch_buffers = T.n_buffers;
-          D.patch_grid = T.grid;
-          PMG_HIP_CHECK(hipStreamSynchronize(c->stream));
-        }
-      }
-      if (D.lu) {
-        if (D.patch_rec) D.patch_alt = dalloc<double>(c, 3 * size_t(D.n_udof) * std::max(1, D.patch_buffers - 1));
-      } else if (D.minv32 || D.minv16) {
-        D.ua32 = dalloc<float>(c, 4 * size_t(D.n_udof) * D.patch_buffers);
+        if (takes_patch_step(c, D)) build_patch_records(c, D, d, ug, pg, reo.data());
       } else if (c->prm.precision == PMG_PREC_FP32) {
         D.lu32 = dalloc<float>(c, lun);
         launch_fill<float>(D.lu32, 0.0f, long(lun), c->stream);

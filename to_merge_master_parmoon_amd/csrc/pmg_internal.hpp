@@ -168,13 +168,13 @@ struct DevLevel {
   uint16_t *minv16 = nullptr;
   // FP32 sweeps with inverses and the shared block: interleaved copy (u1, u2, u3, 0) of the
   // velocity the residual gathers, built at the sweep start and kept by the local updates
-  // With the patch records below it holds patch_buffers such copies, the current one first.
+  // With the patch records below it holds several such copies, the current one first.
   float *ua32 = nullptr;
-  // records of the fused color step (null: the two-launch form)
+  // records of the fused color step (null: the two-launch form); tried: their build was
   int *patch_rec = nullptr;
   uint32_t *patch_pat = nullptr;
-  int patch_stride = 0, patch_buffers = 1;
-  bool patch_grid = false;
+  int patch_stride = 0;
+  bool patch_grid = false, patch_tried = false;
   double *patch_alt = nullptr;       // FP64: the copies of the velocity after the first
   // the patch inverses are stored in the block form (set at every factorization: shared
   // velocity block present)
