@@ -4,11 +4,13 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <deque>
+#include <memory>
 #include <mutex>
-#include <string>
 #include <system_error>
 #include <thread>
 #include <unordered_map>
+#include <utility>
 
 namespace pmg {
 
@@ -51,12 +53,25 @@ bool color_lists(int n_dof, int per_cell, const std::vector<int> &glob, int n_co
   return true;
 }
 
+// hash of a pattern -> its words and its number
+using Patterns = std::unordered_multimap<uint64_t, std::pair<const std::vector<uint32_t> *, int>>;
+
 struct Scratch {
   std::vector<int> mark, pmark;   // dof -> place in the halo (valid where stamp matches)
   std::vector<int> stamp, pstamp;
   std::vector<int> halo, runs;
   std::vector<uint32_t> pat;      // the pattern of the cell in work
+  Patterns seen;                  // those this thread has met
 };
+
+uint64_t pattern_hash(const std::vector<uint32_t> &w) {
+  uint64_t h = w.size();
+  for (size_t i = 0; i + 1 < w.size(); i += 2) {
+    h = (h ^ (w[i] | uint64_t(w[i + 1]) << 32)) * 0x9e3779b97f4a7c15ull;
+    h ^= h >> 32;
+  }
+  return h;
+}
 
 }  // namespace
 
@@ -88,13 +103,10 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
   // local rows by decreasing length into the velocity quads, heaviest wavefronts last filled
   static const int quad_order[7] = {0, 2, 4, 5, 6, 7, 3};
   auto row_places = [&](const int *u, int (&place)[NU]) {
-    int idx[NU];
-    for (int j = 0; j < NU; ++j) idx[j] = j;
-    std::stable_sort(idx, idx + NU, [&](int a, int b) {
-      const int la = len_a(u[a]), lb = len_a(u[b]);
-      return la != lb ? la > lb : len_bt(u[a]) > len_bt(u[b]);
-    });
-    for (int k = 0; k < NU; ++k) place[idx[k]] = quad_order[k / 4] * 4 + k % 4;
+    int key[NU];   // A length, BT length, the lower row first
+    for (int j = 0; j < NU; ++j) key[j] = len_a(u[j]) << 16 | len_bt(u[j]) << 8 | (31 - j);
+    std::sort(key, key + NU, [](int a, int b) { return a > b; });
+    for (int k = 0; k < NU; ++k) place[31 - (key[k] & 31)] = quad_order[k / 4] * 4 + k % 4;
   };
   using G = PatchShape<true>;
   using R = PatchShape<false>;
@@ -121,8 +133,9 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
 
   // records with a fixed largest halo, then packed to the level's own largest halo
   const int wide = PR_HALO + PT_HALO;
-  std::vector<int> rec(size_t(n_pos) * wide, 0);
-  std::unordered_map<std::string, int> known;   // pattern words -> number in the order of arrival
+  std::unique_ptr<int[]> rec(new int[size_t(n_pos) * wide]);   // zeroed by the threads
+  std::deque<std::vector<uint32_t>> known;   // the patterns in the order of arrival (their places stay)
+  Patterns known_at;
   std::mutex known_mu;
   std::atomic<bool> ok{true};
   std::atomic<int> next{0};
@@ -172,6 +185,7 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
         while (nh > h && !hmax.compare_exchange_weak(h, nh)) {
         }
         int *rc = &rec[size_t(q) * wide];
+        std::fill(rc, rc + wide, 0);
         for (int i = 0; i < nh; ++i) {
           const int g = W.halo[i];
           W.mark[g] = i;
@@ -242,9 +256,25 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
           desc(e, k0, 0, n, 0, NU + j, p[j]);
           for (int k = 0; k < n; ++k) put(off_a[1], e, k, n, W.mark[d->b_kcol[k0 + k]]);
         }
-        std::string key(reinterpret_cast<const char *>(W.pat.data()), W.pat.size() * sizeof(uint32_t));
-        std::lock_guard<std::mutex> lk(known_mu);
-        rc[PR_HEAD] = known.emplace(std::move(key), int(known.size())).first->second;
+        // a few hundred patterns among all cells: almost every one is found without the lock
+        const uint64_t hash = pattern_hash(W.pat);
+        auto find = [&](const Patterns &in) {
+          for (auto [it, end] = in.equal_range(hash); it != end; ++it)
+            if (*it->second.first == W.pat) return it->second;
+          return std::pair<const std::vector<uint32_t> *, int>(nullptr, -1);
+        };
+        auto at = find(W.seen);
+        if (!at.first) {
+          std::lock_guard<std::mutex> lk(known_mu);
+          at = find(known_at);
+          if (!at.first) {
+            known.push_back(W.pat);
+            at = {&known.back(), int(known.size()) - 1};
+            known_at.emplace(hash, at);
+          }
+          W.seen.emplace(hash, at);
+        }
+        rc[PR_HEAD] = at.second;
       }
     }
   };
@@ -269,20 +299,18 @@ void build_patch_tables(const pmg_level_desc *d, const std::vector<int> &ug, con
   if (!ok) return;
   // the patterns in the order of their first cell, whatever order the threads met them in
   std::vector<int> number(known.size(), -1);
-  std::vector<const std::string *> text(known.size());
-  for (const auto &kv : known) text[kv.second] = &kv.first;
   T.pat.resize(known.size() * size_t(words));
   for (int q = 0; q < n_pos; ++q) {
     int &id = rec[size_t(q) * wide + PR_HEAD];
     if (number[id] < 0) {
       number[id] = T.n_patterns++;
-      std::memcpy(&T.pat[size_t(number[id]) * words], text[id]->data(), text[id]->size());
+      std::copy(known[id].begin(), known[id].end(), &T.pat[size_t(number[id]) * words]);
     }
     id = number[id];
   }
-  T.stride = (PR_HALO + hmax + 15) / 16 * 16;
-  T.rec.resize(size_t(n_pos) * T.stride);
-  for (int q = 0; q < n_pos; ++q) std::memcpy(&T.rec[size_t(q) * T.stride], &rec[size_t(q) * wide], 4 * std::min(wide, T.stride));
+  T.stride = (PR_HALO + hmax + 15) / 16 * 16;   // at most wide
+  for (int q = 1; q < n_pos; ++q) std::memmove(&rec[size_t(q) * T.stride], &rec[size_t(q) * wide], 4 * size_t(T.stride));
+  T.rec = std::move(rec);
   T.ok = true;
 }
 

@@ -6,6 +6,7 @@
 // where the value from before the color is kept.
 #pragma once
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "pmg.h"
@@ -66,7 +67,7 @@ struct PatchTables {
   int n_buffers = 1;         // copies of the velocity the step alternates between
   int n_patterns = 0;
   bool grid = false;         // the patterns have PatchShape*<true>, else <false>
-  std::vector<int> rec;
+  std::unique_ptr<int[]> rec;   // stride ints per color position
   std::vector<uint32_t> pat;
 };
 

@@ -631,8 +631,9 @@ void build_patch_records(pmg_ctx *c, DevLevel &D, const pmg_level_desc *d, const
   build_patch_tables(d, ug, pg, D.n_colors, D.ptr_colors.data(), order, D.lu != nullptr, T);
   if (!T.ok) return;
   drop_graph(c);   // a captured V-cycle holds the two launches and the old copy
-  int *rec = dalloc<int>(c, T.rec.size());
-  h2d(c, rec, T.rec.data(), T.rec.size());
+  const size_t len = size_t(D.ptr_colors[D.n_colors]) * T.stride;
+  int *rec = dalloc<int>(c, len);
+  h2d(c, rec, T.rec.get(), len);
   D.patch_pat = dalloc<uint32_t>(c, T.pat.size());
   h2d(c, D.patch_pat, T.pat.data(), T.pat.size());
   D.patch_stride = T.stride;
