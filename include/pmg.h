@@ -400,10 +400,11 @@ typedef struct {
 } pmg_timers;
 /* Launch-shape autotuner (no reference counterpart; the reference's kernels have fixed
    shapes): after pmg_setup, times the candidate launch shapes of every smoothed level's
-   kernels on the device, reps launches each, and keeps the fastest per level: work items
-   per workgroup of the Vanka residual (16, 32, 64), whether colors of >= 512 cells run in
-   per-XCD groups, operator rows per workgroup of the type-4 defect / matvec (32 .. 256).
-   The shapes change how work is distributed, not what is computed (only the summation
+   kernels on the device, reps launches each, and keeps the fastest per level: whether colors
+   of >= 512 cells run in per-XCD groups, work items per workgroup of the Vanka residual
+   where a sweep launches it by itself (16, 32, 64; FP64 levels always, for
+   pmg_vanka_smooth_noalloc), operator rows per workgroup of the type-4 defect / matvec (16 ..
+   256, or 0 unless one of them is faster by 2 %).  The shapes change how work is distributed, not what is computed (only the summation
    order of the pressure means differs).  Uses the levels' own work vectors.
    pmg_level_tuning returns {residual items per workgroup FP64, FP32; XCD groups FP64,
    FP32; operator rows per workgroup FP64, FP32} (0: built-in default). */

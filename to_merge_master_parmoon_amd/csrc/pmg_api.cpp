@@ -688,6 +688,33 @@ float *sweep_copy(const pmg_ctx *c, const DevLevel &D) {
   return nullptr;
 }
 
+// One launch per color: residual, local solve and update of a patch by one workgroup, at every
+// size faster than the two launches (k_patch.hip); these stay for refinement steps, nine
+// blocks in FP64 or off a hexahedral grid, stored FP32 LU factors and levels whose patches fit
+// no record (rows of more than 128 entries, shared pressure dofs, colors that share dofs).
+// ua: sweep_copy of the level
+template <typename T>
+bool takes_fused(const pmg_ctx *c, const DevLevel &D, const float *ua) {
+  if (sizeof(T) == 8) return D.patch_rec && D.a_shared;
+  return ua && D.patch_rec && c->prm.bf16_refine_steps == 0;
+}
+// nc patches of the color whose positions start at p0; xcd: in groups per XCD
+template <typename T>
+void launch_fused(pmg_ctx *c, DevLevel &D, int p0, int nc, const int *slots, T *u, const T *f, float *ua, T damp,
+                  bool xcd) {
+  const OpView<T> op = opview<T>(D);
+  if constexpr (sizeof(T) == 4) {
+    const bool full = !D.schur;
+    PatchStep P{D.patch_rec, D.patch_pat, slots, op.a1, op.btv, op.bv, f, u, ua, damp, D.patch_stride, D.n_udof,
+                nc, p0, xcd, full, D.patch_grid, D.a_shared ? nullptr : op.av, D.invperm, op.n_active};
+    launch_patch_step(P, D.minv32, D.minv16, full, c->stream);
+  } else {
+    PatchStep64 P{D.patch_rec, D.patch_pat, slots, D.invperm, op.a1, op.btv, op.bv, f, D.lu, u, D.patch_alt, damp,
+                  D.patch_stride, D.n_udof, nc, p0, xcd, D.patch_grid};
+    launch_patch_step64(P, c->stream);
+  }
+}
+
 template <typename T>
 // last = false: another sweep with the same f follows at once and sets the Dirichlet values
 // again before anything reads them, so this sweep's closing SetDirichletNodes is left out
@@ -730,12 +757,7 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
   if (relax) launch_copy<T>(aux, u, D.n_dof, c->stream);
   const OpView<T> op = opview<T>(D);
   const int nref = sizeof(T) == 4 ? c->prm.bf16_refine_steps : 0;
-  // one launch per color: residual, local solve and update of a patch by one workgroup, at every
-  // size faster than the two launches (k_patch.hip); these stay for refinement steps, nine
-  // blocks in FP64 or off a hexahedral grid, stored FP32 LU factors and levels whose patches fit
-  // no record (rows of more than 128 entries, shared pressure dofs, colors that share dofs)
-  const bool fused = sizeof(T) == 8 ? rloc == reinterpret_cast<T *>(D.rloc) && D.patch_rec && D.a_shared
-                                    : ua && D.patch_rec && nref == 0;
+  const bool fused = takes_fused<T>(c, D, ua) && (sizeof(T) == 4 || rloc == reinterpret_cast<T *>(D.rloc));
   const bool full = !D.schur;
   for (int col = 0; col < D.n_colors; ++col) {
     const int p0 = D.ptr_colors[col];
@@ -755,26 +777,15 @@ void vanka_sweep(pmg_ctx *c, DevLevel &D, T *u, const T *f, T *aux, T *rloc, boo
       nc = int(D.act_slots_off[col + 1] - D.act_slots_off[col]);
       if (nc == 0) continue;
     }
-    if constexpr (sizeof(T) == 4) {
-      if (fused) {
-        const double sb = full ? double(MINV_STRIDE) : double(SCH_STRIDE);
-        // the rows of the residual, the stored data, the record, the new values
-        const double by = (D.res_bytes[D.a_shared][1][col] - D.res_index_bytes[col]) * part - nc * (31.0 * 20 + 2 * 85 * 4.0) +
-                          nc * (sb * fb + 4.0 * D.patch_stride + 27 * 16.0 + 32);
-        Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
-        PatchStep P{D.patch_rec, D.patch_pat, slots, op.a1, op.btv, op.bv, f, u, ua, damp, D.patch_stride, D.n_udof,
-                    nc, p0, nc >= XCD_GROUP_MIN && D.tune_res_xcd[1], full, D.patch_grid, D.a_shared ? nullptr : op.av,
-                    D.invperm, op.n_active};
-        launch_patch_step(P, D.minv32, D.minv16, full, c->stream);
-        continue;
-      }
-    } else if (fused) {
-      const double by = (D.res_bytes[1][0][col] - D.res_index_bytes[col]) * part - nc * (31.0 * 20 + 85 * 8.0) +
-                        nc * (NLOC * NLOC * 8.0 + 4.0 * D.patch_stride + 85 * 8.0);
+    if (fused) {
+      // the rows of the residual, the stored data, the record, the new values
+      const int pi = sizeof(T) == 8 ? 0 : 1;
+      const double sb = pi == 0 ? NLOC * NLOC * 8.0 : (full ? double(MINV_STRIDE) : double(SCH_STRIDE)) * fb;
+      const double by = (D.res_bytes[D.a_shared][pi][col] - D.res_index_bytes[col]) * part -
+                        nc * (31.0 * 20 + (pi == 0 ? 85 * 8.0 : 2 * 85 * 4.0)) +
+                        nc * (sb + 4.0 * D.patch_stride + (pi == 0 ? 85 * 8.0 : 27 * 16.0 + 32));
       Timed tm(c, &c->tm.vanka_res, by, nc * 2.0 * NLOC * NLOC, &D == &c->L.back() ? &c->tm.vanka_res_finest : nullptr);
-      PatchStep64 P{D.patch_rec, D.patch_pat, slots, D.invperm, op.a1, op.btv, op.bv, f, D.lu, u, D.patch_alt, damp,
-                    D.patch_stride, D.n_udof, nc, p0, nc >= XCD_GROUP_MIN && D.tune_res_xcd[0], D.patch_grid};
-      launch_patch_step64(P, c->stream);
+      launch_fused<T>(c, D, p0, nc, slots, u, f, ua, damp, nc >= XCD_GROUP_MIN && D.tune_res_xcd[pi]);
       continue;
     }
     {
@@ -858,7 +869,7 @@ OpView<double> op64_for(pmg_ctx *c, const DevLevel &D, const double *x) {
   }
   return o;
 }
-OpView<float> op64_for(pmg_ctx *, const DevLevel &D, const float *) { return D.op32(); }
+OpView<float> op64_for(pmg_ctx *, const DevLevel &D, const float *) { return D.op32(); }   // no copy in FP32
 
 // res_dev (single problem only): ||d||_2 after the projection
 template <typename T>
@@ -2546,9 +2557,10 @@ int pmg_vanka_smooth(pmg_ctx *c, int level, double *u, const double *f, int nswe
 // ------------------------------------------------------------------ launch-shape autotuner
 // Times the candidate launch shapes of the level kernels on the device (HIP events around
 // `reps` launches each, after one untimed launch) and keeps the fastest per level and
-// precision: work items per workgroup of the Vanka residual (16, 32, 64), whether large
-// colors run in their per-XCD groups, and operator rows per workgroup of the type-4
-// kernels (32 .. 256).  Every candidate computes the same values (the work is only
+// precision: whether large colors run in their per-XCD groups (of the one-launch color step where
+// the level takes it), work items per workgroup of the Vanka residual where it is launched by
+// itself (16, 32, 64), and operator rows per workgroup of the type-4 kernels (16 .. 256, or the
+// built-in rule), with the interleaved input where the calls make one.  Every candidate computes the same values (the work is only
 // distributed differently), so the choice changes timings, not results, except for the
 // summation order of the grid-wide pressure reductions.
 extern "C++" {
@@ -2595,17 +2607,17 @@ static void tune_level(pmg_ctx *c, DevLevel &D, int reps, bool finest) {
   if (D.n_colors > 0 && !D.nodal) {
     float *ua = nullptr;
     if constexpr (sizeof(T) == 4) {
-      if (D.ua32 && D.a_shared && (D.minv16 || D.minv32)) {
-        ua = D.ua32;
-        launch_sweep_start(u, f, D.n_udof, D.hanging_bound, D.n_dirichlet, ua, c->stream);
-      }
+      ua = sweep_copy<T>(c, D);
+      if (ua) launch_sweep_start(u, f, D.n_udof, D.hanging_bound, D.n_dirichlet, ua, c->stream);
     }
-    const bool grouped = D.h_xcd_grouped[0];
+    const bool fused = takes_fused<T>(c, D, ua);
+    // large colors: in their groups per XCD or not
+    const bool grouped = fused ? D.max_cells_per_color >= XCD_GROUP_MIN : bool(D.h_xcd_grouped[0]);
     T *uloc = sizeof(T) == 4 ? reinterpret_cast<T *>(D.uloc32) : nullptr;
-    // one pass = the residual launches of every color in sweep order (each color reads its
+    // one pass = the launches of every color in sweep order (each color reads its
     // own rows, as in a sweep; one color repeated would find its rows in the caches)
     const int passes = std::max(1, reps / std::max(1, D.n_colors));
-    auto pass = [&](int xcd, int pb) {
+    auto residuals = [&](int xcd, int pb) {
       for (int col = 0; col < D.n_colors; ++col) {
         const int p0 = D.ptr_colors[col];
         const long n_items = long(D.ptr_colors[col + 1] - p0) * (NU_LOC + NP_LOC);
@@ -2615,18 +2627,33 @@ static void tune_level(pmg_ctx *c, DevLevel &D, int reps, bool finest) {
         launch_vanka_residual<T>(op, n_items, p0, D.invperm, items, desc, xg, u, ua, f, rloc, uloc, c->stream, pb);
       }
     };
+    auto steps = [&](int xcd) {   // with a damping of zero: u stays as it is
+      for (int col = 0; col < D.n_colors; ++col) {
+        const int p0 = D.ptr_colors[col], nc = D.ptr_colors[col + 1] - p0;
+        launch_fused<T>(c, D, p0, nc, nullptr, u, f, ua, T(0), xcd && nc >= XCD_GROUP_MIN);
+      }
+    };
     // three rounds over the candidates, each candidate's fastest round counts (the rounds
     // interleave the candidates, so a slow phase of the device does not favour one)
-    std::vector<std::pair<int, int>> cand;
-    for (int xcd = grouped ? 0 : 1; xcd <= 1; ++xcd)
-      for (int pb : {16, 32, 64}) cand.emplace_back(xcd, pb);
-    std::vector<float> best(cand.size(), 1e30f);
-    for (int round = 0; round < 3; ++round)
-      for (size_t k = 0; k < cand.size(); ++k)
-        best[k] = std::min(best[k], time_launches(c, passes, [&] { pass(cand[k].first, cand[k].second); }));
-    const size_t kb = size_t(std::min_element(best.begin(), best.end()) - best.begin());
-    D.tune_res_xcd[pi] = cand[kb].first;
-    D.tune_res_pb[pi] = cand[kb].second;
+    auto fastest = [&](const std::vector<std::pair<int, int>> &cand, auto &&pass) {
+      std::vector<float> best(cand.size(), 1e30f);
+      for (int round = 0; round < 3; ++round)
+        for (size_t k = 0; k < cand.size(); ++k)
+          best[k] = std::min(best[k], time_launches(c, passes, [&] { pass(cand[k].first, cand[k].second); }));
+      return cand[size_t(std::min_element(best.begin(), best.end()) - best.begin())];
+    };
+    if (fused && grouped) D.tune_res_xcd[pi] = fastest({{0, 0}, {1, 0}}, [&](int xcd, int) { steps(xcd); }).first;
+    // the residual of its own: where the sweep launches it (a fused FP64 level's
+    // pmg_vanka_smooth_noalloc does, with the step's XCD flag)
+    if (!fused || sizeof(T) == 8) {
+      std::vector<std::pair<int, int>> cand;
+      for (int xcd = 0; xcd <= 1; ++xcd)
+        for (int pb : {16, 32, 64})
+          if (fused || !grouped ? xcd == D.tune_res_xcd[pi] : true) cand.emplace_back(xcd, pb);
+      const std::pair<int, int> k = fastest(cand, residuals);
+      D.tune_res_xcd[pi] = k.first;
+      D.tune_res_pb[pi] = k.second;
+    }
   }
   // the MG defect of this level (and, finest level of a mixed context, the FP64 matvec)
   auto tune_op = [&](auto zero, int mode, int slot) {
@@ -2636,17 +2663,18 @@ static void tune_level(pmg_ctx *c, DevLevel &D, int reps, bool finest) {
       launch_fill<U>(x, U(0.5), D.n_dof, c->stream);
       launch_fill<U>(b, U(1.0), D.n_dof, c->stream);
     }
-    const int cand[4] = {32, 64, 128, 256};
-    float best[4] = {1e30f, 1e30f, 1e30f, 1e30f};
+    // 0: the built-in rule, kept unless another shape is faster by 2 %
+    const int cand[6] = {0, 16, 32, 64, 128, 256};
+    float best[6] = {1e30f, 1e30f, 1e30f, 1e30f, 1e30f, 1e30f};
     for (int round = 0; round < 3; ++round)
-      for (int k = 0; k < 4; ++k) {
-        OpView<U> o = opview<U>(D);
-        o.rpb = cand[k];
+      for (int k = 0; k < 6; ++k)
         best[k] = std::min(best[k], time_launches(c, reps, [&] {
+          OpView<U> o = op64_for(c, D, x);
+          o.rpb = cand[k];
           launch_type4<U>(o, mode, x, b, yy, mode != 0 && fused_l20(c), nullptr, c->red, c->stream);
         }));
-      }
-    D.tune_op_rpb[slot] = cand[std::min_element(best, best + 4) - best];
+    const int kb = int(std::min_element(best, best + 6) - best);
+    D.tune_op_rpb[slot] = best[kb] < 0.98f * best[0] ? cand[kb] : 0;
   };
   tune_op(T(0), 2, pi);
   if (finest && pi == 1) tune_op(double(0), 0, 0);
@@ -2658,6 +2686,7 @@ int pmg_autotune(pmg_ctx *c, int reps) {
   return guard(c, [&] {
     PMG_NEED_READY();
     drop_graph(c);
+    ensure_xa(c);
     const bool mx = mixed(c);
     // the coarsest level is solved directly (no smoother, no defect in the cycle)
     for (size_t l = 1; l < c->L.size(); ++l) {
