@@ -7,6 +7,8 @@ Pins:
   * (gpu) re-assembling every level with the generator's own convection values, viscosity
     and mass term reproduces the operator the generator assembled on the host, on perturbed
     cubes and on the channel step system (matvec of random vectors, 1e-13);
+  * (gpu) the matrix-free right-hand side of the theta scheme without its mass term is minus that host
+    operator times the velocity, on perturbed boxes of 1 to 512 cells (1e-13);
   * (gpu) the velocity at the Gauss points of the Q2 interpolant of a global quadratic field
     equals the field at the mapped Gauss points (Q2 on trilinear cells holds such fields);
   * (gpu) fixed-point (Picard) steps with convection b = u_k re-assembled on the device
@@ -73,6 +75,30 @@ def test_reassembly_reproduces_host_operator(case):
         y1 = mg.matvec(l, x)
         print(case, "level", l, "rel", rel(y1, y0), flush=True)
         assert rel(y1, y0) <= 1e-13
+    mg.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("box", [(1, 1, 1), (3, 1, 2), (4, 4, 4)])
+def test_theta_rhs_matches_host_operator(box):
+    from to_merge_master_parmoon_amd import _abi, problem
+    from to_merge_master_parmoon_amd.multigrid import DeviceVector
+    p = problem.Problem(cx=box[0], cy=box[1], cz=box[2], n_levels=2, nu=0.02, conv_kind=_abi.CONV_FOURIER,
+                        rhs_kind=_abi.RHS_FOURIER, dirichlet_faces=problem.DIRICHLET_X0_Y0_Z0, perturb=0.1)
+    mg = _hier_with_geometry(p, internal_project_pressure=0)
+    rng = np.random.default_rng(13)
+    for l in range(p.n_levels):
+        d, n = p.descs[l], mg.n_dof[l]
+        u, g = rng.standard_normal(n), rng.standard_normal(n)
+        uv, gv, rv = DeviceVector(mg, n, u), DeviceVector(mg, n, g), DeviceVector(mg, n, rng.standard_normal(n))
+        bq = DeviceVector(mg, 81 * d.n_cells, p.conv_quad(l).reshape(-1))
+        mg._check(mg._lib.pmg_theta_rhs(mg._ctx, l, uv.ptr, bq.ptr, 0.02, 0.0, gv.ptr, rv.ptr, 1))
+        u[3 * d.n_udof:] = 0.0
+        want = -mg.matvec(l, u)   # the host operator's rows
+        want[3 * d.n_udof:] = 0.0
+        for c in range(3):
+            want[c * d.n_udof + d.n_active:(c + 1) * d.n_udof] = g[c * d.n_udof + d.n_active:(c + 1) * d.n_udof]
+        assert rel(rv.download(), want) <= 1e-13
     mg.close()
 
 

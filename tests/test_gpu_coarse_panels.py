@@ -2,7 +2,8 @@
 substitution with the factors read from memory), at the edges of its range: 512 unknowns
 (still the one-workgroup LU), 567 and 640, 729 and 1000 (the 5^3 grids), 1008 with 504 pressures.
 Against the FP64 form's LU of the whole reduced system, which matches the oracle's
-dgetrf/dgetrs; both solve the same system in FP64, 1e-10 as for the smaller blocks."""
+dgetrf/dgetrs; both solve the same system in FP64, 1e-10 as for the smaller blocks.  Twice, the second
+time with other values in the same buffers."""
 import numpy as np
 import pytest
 
@@ -25,16 +26,17 @@ def test_panel_block_coarse_solve(box, faces, m):
     for precision in (0, 1, 2):
         mg = build_hierarchy(prob, params(precision=precision, **prm))
         out.append(mg.solve_exact(f))
-        if precision:   # a second operator in the same buffers
-            a = prob.arrays(0)
-            for v in a["a"]:
-                v *= 1.25
-            mg.update_values(0, prob.descs[0])
-            mg.refactor()
-            out[-1] = np.concatenate([out[-1], mg.solve_exact(f)])
-            for v in a["a"]:
-                v *= 0.8
+        # a second operator in the same buffers, the reference's LU again beside the block form
+        keep = [v.copy() for v in prob.arrays(0)["a"]]
+        for v in prob.arrays(0)["a"]:
+            v *= 1.25
+        mg.update_values(0, prob.descs[0])
+        mg.refactor()
+        out[-1] = np.concatenate([out[-1], mg.solve_exact(f)])
+        for v, k in zip(prob.arrays(0)["a"], keep):
+            v[:] = k
         mg.close()
     n = len(f)
-    assert rel(out[1][:n], out[0]) <= 1e-10 and rel(out[2][:n], out[0]) <= 1e-10
-    assert rel(out[1][n:], out[2][n:]) <= 1e-10 and rel(out[1][n:], out[0]) > 1e-3
+    for x in out[1:]:
+        assert rel(x[:n], out[0][:n]) <= 1e-10 and rel(x[n:], out[0][n:]) <= 1e-10
+    assert rel(out[0][n:], out[0][:n]) > 1e-3

@@ -1,7 +1,8 @@
 """One launch per color with nine velocity blocks (csrc/k_patch.hip): FP32 and BF16 sweeps against the
 oracle's FP64 sweep on boxes one coarse cell wide, colors of 1 to 8 cells, and faces with
-Dirichlet rows whose coupling blocks hold values that the sweep has to drop; then the same level
-with refinement steps, which take the two launches.  Bounds: FP32 rounding of the local
+Dirichlet rows whose coupling blocks hold values that the sweep has to drop, without and with the
+global relaxation (each sweep then starts from a velocity that the one before did not leave); then
+the same level with refinement steps, which take the two launches.  Bounds: FP32 rounding of the local
 inverses 2e-5, BF16's 2e-2, as with the shared block."""
 import numpy as np
 import pytest
@@ -12,8 +13,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("box,faces", [((1, 1, 1), 1), ((1, 1, 3), 21), ((3, 2, 2), 63), ((4, 4, 1), 21)])
-@pytest.mark.parametrize("precision,refine,bound", [(1, 0, 2e-5), (2, 0, 2e-2), (2, 1, 2e-2)])
-def test_nine_block_color_step(box, faces, precision, refine, bound):
+@pytest.mark.parametrize("precision,refine,alpha,bound", [(1, 0, 1.0, 2e-5), (2, 0, 1.0, 2e-2), (2, 1, 1.0, 2e-2),
+                                                          (1, 0, 0.8, 2e-5), (2, 0, 0.8, 2e-2)])
+def test_nine_block_color_step(box, faces, precision, refine, alpha, bound):
     import pmg_oracle
     from to_merge_master_parmoon_amd import _abi, problem
     from to_merge_master_parmoon_amd.multigrid import NSEMultiGrid
@@ -28,7 +30,7 @@ def test_nine_block_color_step(box, faces, precision, refine, bound):
             a[b][:ne] = w * a0
             a[b][ne:] = rng.standard_normal(len(a[b]) - ne)
         a[4][:ne] = 1.1 * a0
-    prm = dict(internal_project_pressure=1 if faces == 63 else 0)
+    prm = dict(internal_project_pressure=1 if faces == 63 else 0, sc_smooth_damp_factor_saddle=alpha)
     u = rng.standard_normal(prob.n_dof(1))
     f = rng.standard_normal(prob.n_dof(1))
     orc = pmg_oracle.Oracle(params(**prm), prob.descs, refactor=0)

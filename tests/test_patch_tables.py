@@ -1,7 +1,7 @@
 """The per-cell records of the fused Vanka color step (csrc/patch_tables.cpp), on the CPU:
 tests/patch_driver.cpp runs colored sweeps from the records on generated levels (cubes, open
 and one-cell-wide boxes, greedy colors, Gauss-Seidel level sets, colorings that leave cells
-out), patches of a color in random order, and compares them with the sweep from its
+out, rows longer than a hexahedral grid's), patches of a color in random order, and compares them with the sweep from its
 definition (double sums of at most 128 terms in another order: 1e-12)."""
 import shutil
 import subprocess
@@ -24,4 +24,5 @@ def test_sweeps_from_records(tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.strip().endswith("OK"), r.stdout
     assert " 3 buffers" in r.stdout   # dofs with an odd number of updates were among them
+    assert ", general," in r.stdout   # and rows longer than a hexahedral grid's
     print(r.stdout)

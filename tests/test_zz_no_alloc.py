@@ -2,8 +2,8 @@
 pmg_vanka_smooth for callers that cannot allocate, with their scratch in a file-scope
 device array) against pmg_vanka_smooth, through the C ABI on device vectors.
 
-The two entry points run the same kernels on the same inputs, so their results are
-compared bit for bit, on two calls in a row with the second on a smaller level (the array
+pmg_vanka_smooth takes one launch per color and the other the residual and the local solve in two,
+with the same arithmetic, so their results are compared bit for bit, on two calls in a row with the second on a smaller level (the array
 keeps the first call's contents), with the global relaxation on (its copy of u lives in
 the array too) and off; a level whose scratch exceeds the array is refused with
 PMG_ERR_UNSUPPORTED, as is a mixed-precision context.
