@@ -381,7 +381,7 @@ __global__ void k_coarse_out(OpView<double> op, const double *__restrict__ f, co
 // each, stored and polled by relaxed 64-bit atomics, so a hop is one store and one load (a flag
 // beside the data took a release, which writes back the XCD's L2, and an acquire per poll).  The
 // steps have no select in the chain: entries that a step does not use are zero.  1284 unknowns:
-// forward 138 -> 47 us, backward 155 -> 53 us, the same sums in the same order.
+// forward 138 -> 48 us, backward 155 -> 56 us, the same sums in the same order.
 constexpr long SPIN_LIMIT = 1L << 24;
 
 template <bool UPPER>
@@ -469,15 +469,15 @@ __global__ __launch_bounds__(256) void k_trsv_chain(const double *__restrict__ f
     }
     z = quotient(z);
     // unless one of the unknowns is not finite, which zero times it would carry to the finished rows
-    // (and which its own row shows at the end): again with selects
-    if (__any(r < kb && !(fabs(z) < INFINITY))) {
+    // (and which its own row shows at the end): again with selects.  (The upper sweep only: one in
+    // the lower sweep makes all later rows and, from the last row's quotient on, all unknowns NaN.)
+    if (UPPER && __any(r < kb && !(fabs(z) < INFINITY))) {
       z = v;
 #pragma unroll 1
-      for (int i = 0; i < kb; ++i) {
-        const int k = UPPER ? kb - 1 - i : i;
+      for (int k = kb - 1; k >= 0; --k) {
         const double q = quotient(z), xk = bcast(q, k);
         if (r == k) z = q;
-        if (r < kb && (UPPER ? r < k : r > k)) z = fma(-xk, f[long(R0 + k) * n + row], z);
+        if (r < k) z = fma(-xk, f[long(R0 + k) * n + row], z);
       }
     }
     if (r < kb) {
@@ -592,7 +592,10 @@ void launch_coarse_build(const DevLevel &L, Coarse &C, hipStream_t s) {
 
 // a (n x n, row-major) := L U by panels, sigma[i] = original row now at row i
 void lu_factor_panels(double *a, int n, int *ipiv, int *sigma, double *ubuf, int *swp, int *info, hipStream_t s) {
-  const int pr_max = 7;   // PR = 7 spills 16 VGPRs to scratch; 8 would spill ~1000
+  // PR = 7 (512 threads, the first panels of 3073 unknowns and more) spills 286 registers, 92 B of
+  // scratch a lane, and takes 124 us as with the pivot search by shuffles, which spilled 16; PR = 6
+  // and fewer spill none and went from 98 to 86 us (6) .. 41 to 24 us (1)
+  const int pr_max = 7;
   if ((n + PNT - 1) / PNT > pr_max)
     throw DeviceError("coarse system of " + std::to_string(n) + " unknowns exceeds the dense LU limit (" +
                       std::to_string(pr_max * PNT) + ")");

@@ -9,7 +9,9 @@
 // at its step instead costs 3 % of a color).  FP64, one color of the fused step (k_patch.hip): 8^3
 // 11.6 -> 9.2 us, 16^3 17.7 -> 15.8 us, the same results bit for bit.
 // An unknown that is not finite would come to the rows that its column does not reach as zero
-// times it.  Its own row shows it at the end; the sweep is then run again with selects.
+// times it.  Its own row shows it at the end; the sweep is then run again with selects.  (In FP64 the
+// upper sweep only: one in the lower sweep makes all later rows and, from the last row's quotient
+// on, all unknowns NaN with selects too.)
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -94,7 +96,7 @@ __device__ __forceinline__ void lower_sweep(const F *s, int lane, T &x0, T &x1) 
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (!any_not_finite(lane, x0, x1)) return;
+  if (sizeof(T) == 8 || !any_not_finite(lane, x0, x1)) return;
   x0 = r0;
   x1 = r1;
 #pragma unroll 1
