@@ -404,8 +404,9 @@ typedef struct {
    of >= 512 cells run in per-XCD groups, work items per workgroup of the Vanka residual
    where a sweep launches it by itself (16, 32, 64; FP64 levels always, for
    pmg_vanka_smooth_noalloc), operator rows per workgroup of the type-4 defect / matvec (16 ..
-   256, or 0 unless one of them is faster by 2 %).  The shapes change how work is distributed, not what is computed (only the summation
-   order of the pressure means differs).  Uses the levels' own work vectors.
+   256, or 0 unless one of them is faster by 2 %).  The shapes change how work is
+   distributed, not what is computed (only the summation order of the pressure means
+   differs).  Uses the levels' own work vectors.
    pmg_level_tuning returns {residual items per workgroup FP64, FP32; XCD groups FP64,
    FP32; operator rows per workgroup FP64, FP32} (0: built-in default). */
 int  pmg_autotune(pmg_ctx *ctx, int reps);

@@ -61,7 +61,12 @@ constexpr int KREF_FULL = 7232;     // 85 * 85 = 7225, padded
 constexpr int KREF_BT = 729, KREF_B = 729 + 324;
 // nodal Vanka: velocity dofs of one B row (27 for Q2/P1disc), upper bound
 constexpr int NODAL_MAXU = 28;
-// colors of at least this many cells run their residual items in 8 per-XCD groups
+// colors of at least this many cells run in 8 per-XCD groups: the residual's items, and the patches
+// of the one-launch color step.  The step with and without them, us per color of a sweep (BF16 /
+// FP32 / FP64): 64 cells 6.0, 6.0 / 6.1, 6.1 / 10.1, 10.1; 288 cells 6.7, 6.9 / 7.4, 7.5 / 14.1, 14.7;
+// 512 cells 6.8, 7.4 / 7.6, 8.1 / 16.4, 17.5; 1000 cells 9.5, 11.1 / 12.2, 13.6 / 27.6, 28.8; 4096 cells
+// 21.2, 27.5 / 23.4, 29.5 / 93.7, 92.1 (the factors fill the caches).  They win by 2 to 5 % from
+// about 300 cells on; the line is where the residual's items had it
 constexpr int XCD_GROUP_MIN = 512;
 static_assert(PM_NB + NP_LOC <= PM_STRIDE, "patch map stride");
 
