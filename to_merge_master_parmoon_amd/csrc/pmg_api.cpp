@@ -2442,6 +2442,7 @@ int pmg_level_update_values(pmg_ctx *c, int level, const pmg_level_desc *d) {
     DevLevel &D = level_of(c, level);
     if (d->a_nnz != D.a_nnz || d->b_nnz != D.b_nnz || d->bt_nnz != D.bt_nnz)
       throw Fail{PMG_ERR_INVALID_ARGUMENT, "pattern changed"};
+    PMG_HIP_CHECK(hipStreamSynchronize(c->stream2));   // the coarse LU may still read the values
     upload_values(c, D, d);
     D.factors_ready = false;
     if (level == 0) c->coarse.ready = false;
